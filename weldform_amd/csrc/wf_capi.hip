@@ -622,10 +622,24 @@ void allocate(Ctx *c) {
     d.ngroups = ng;
     d.gzone = c->gsum_zone;
     d.ghist_cap = c->gsum_cap;
-    d.goff = c->alloc<int>(off.size());
     d.gidx = c->alloc<int>(idx.size());
-    dput(c, d.goff, off);
     dput(c, d.gidx, idx);
+    // (an empty group keeps one empty chunk, which writes its zeros)
+    std::vector<int4> chunk;
+    std::vector<int> nch(ng);
+    for (int g = 0; g < ng; ++g) {
+      const int first = (int)chunk.size();
+      for (int b = off[g]; b < off[g + 1] || b == off[g]; b += kGroupChunk)
+        chunk.push_back(make_int4(g, b, std::min(b + kGroupChunk, off[g + 1]), first));
+      nch[g] = (int)chunk.size() - first;
+    }
+    d.ngchunks = (int)chunk.size();
+    d.gchunk = c->alloc<int4>(chunk.size());
+    d.gnch = c->alloc<int>(ng);
+    d.gticket = c->alloc<int>(ng);
+    d.gpart = c->alloc<double>(chunk.size() * kMaxMesh * 3);
+    dput(c, d.gchunk, chunk);
+    dput(c, d.gnch, nch);
     d.gr_hist = c->alloc<double>((size_t)d.ghist_cap * ng * 3);
     if (d.contact) {
       d.gcf = c->alloc<double4>((size_t)kMaxMesh * np);

@@ -84,6 +84,22 @@ __device__ inline void combine_lanes(R (&v)[NV], R *red) {
   }
 }
 
+// Values handed from block to block inside one launch: written through to
+// the memory the 8 XCDs share (their L2 caches are not coherent with each
+// other) and read past the caches.  The writing wavefront calls stores_done()
+// before it (or, after a barrier, another thread of its block) raises the
+// counter that announces them.  A __threadfence() in its place writes the
+// whole L2 back, which costs tens of microseconds.
+template <typename T>
+__device__ inline void put_agent(T *p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ inline T get_agent(const T *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // ---------------------------------------------------------------------------
 // kernel functions (Source/Functions.cpp:74-87) and the neighbour predicate
 

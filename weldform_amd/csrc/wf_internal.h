@@ -58,6 +58,7 @@ constexpr int kMaxBc = 8;        // velocity / temperature BC slots per context
 constexpr int kMaxZones = 8;     // velocity-BC zones with a reaction history
 constexpr int kMaxMesh = 4;      // rigid contact planes
 constexpr int kMaxContact = 32;  // contact partners per particle
+constexpr int kGroupChunk = 2048;  // particles per block of the per-group sums
 constexpr int kMaxMat = 256;
 constexpr int kMaxNb = 128;
 
@@ -291,12 +292,20 @@ struct Dev {
   double4 *cforce;
   double *cf_hist;             // [hist_cap][kMaxMesh][3]
   // sums per particle group (material index, wf_set_group_sums): each
-  // group's particles in internal order (goff, gidx), per step the reaction
+  // group's particles in internal order (gidx, group after group), per step the reaction
   // of velocity-BC zone gzone (sum m a at the observer) and the contact force
   // of each rigid mesh on the group, kept for the last ghist_cap steps
   int ngroups, gzone;
   long long ghist_cap;
-  int *goff, *gidx;
+  int *gidx;
+  // the groups cut into chunks of at most kGroupChunk particles, one block
+  // each: (group, first and last + 1 place in gidx, the group's first chunk);
+  // gnch chunks per group, gticket counts the finished ones (0 between
+  // launches), gpart their sums [ngchunks][kMaxMesh][3]
+  int ngchunks;
+  int4 *gchunk;
+  int *gnch, *gticket;
+  double *gpart;
   double4 *gcf;                // [kMaxMesh][npad] a particle's contact force per mesh (where ccnt > 0)
   double *gr_hist;             // [ghist_cap][ngroups][3]
   double *gc_hist;             // [ghist_cap][ngroups][kMaxMesh][3]

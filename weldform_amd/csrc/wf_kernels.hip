@@ -2982,51 +2982,89 @@ void launch_force2233(const Dev &d, hipStream_t st, int cur, double xsph, int sh
     k_force2233<false><<<d.nblocks, kBlock, 0, st>>>(d, cur, xsph, shepard);
 }
 
-// Per-group sums (wf_set_group_sums): one block per group walks the group's
-// particles in internal order (thread t takes every kGroupThreads-th) and
-// reduces in a fixed order, so the sums are deterministic.  what 0: the
-// reaction of zone gzone, sum of m a over the group's particles carrying
-// that id, read where the zone reactions are (after the acceleration pass,
-// before contact and the BCs); what 1: the contact force each rigid mesh
-// exerts on the group (after contact).
+// Per-group sums (wf_set_group_sums).  what 0: the reaction of zone gzone,
+// sum of m a over the group's particles carrying that id, read where the
+// zone reactions are (after the acceleration pass, before contact and the
+// BCs); what 1: the contact force each rigid mesh exerts on the group (after
+// contact).  A block sums one chunk of at most kGroupChunk particles (thread
+// t takes every kGroupThreads-th, all of a thread's loads in flight); the
+// block of a group that finishes last (a ticket counter, reset by it) adds
+// the group's chunk sums in chunk order, so the sums are deterministic.
+//
+// The pass reads 8 bytes per particle and is bound by the latency of its two
+// dependent loads.  One block per group walking all of it left 64 blocks on
+// the chip: 183 us per step for 64 groups of 9.4 thousand particles and two
+// meshes; with chunks 18 us (30 us with a fence before the ticket).
 constexpr int kGroupThreads = 256;
+constexpr int kGroupPer = kGroupChunk / kGroupThreads;
 __global__ __launch_bounds__(kGroupThreads) void k_group_sums(Dev d, int what) {
-  __shared__ double sh[kGroupThreads / 64];
-  const int g = blockIdx.x;
-  const long long slot = (d.flags->step % d.ghist_cap) * d.ngroups + g;
-  const int b = d.goff[g], e = d.goff[g + 1];
-  if (what == 0) {
-    double s[3] = {0, 0, 0};
-    for (int p = b + threadIdx.x; p < e; p += kGroupThreads) {
-      const int i = d.gidx[p];
-      if (d.id[i] != d.gzone) continue;
-      const double4 a = d.acc[i];
-      const double m = d.vm[i].w;
-      s[0] += m * a.x, s[1] += m * a.y, s[2] += m * a.z;
-    }
-    for (int k = 0; k < 3; ++k) {
-      const double r = block_reduce<0>(s[k], sh);
-      if (threadIdx.x == 0) d.gr_hist[slot * 3 + k] = r;
-    }
-  } else {
-    for (int m = 0; m < d.nmesh; ++m) {
+  __shared__ double sh[kGroupThreads / 64][3 * kMaxMesh];
+  __shared__ int last;
+  const int4 ch = d.gchunk[blockIdx.x];
+  const int g = ch.x, nm = what == 0 ? 1 : d.nmesh, tid = threadIdx.x;
+  int idx[kGroupPer];
+  bool on[kGroupPer], any = false;
+#pragma unroll
+  for (int u = 0; u < kGroupPer; ++u) {
+    const int p = ch.y + u * kGroupThreads + tid;
+    on[u] = p < ch.z;
+    idx[u] = on[u] ? d.gidx[p] : 0;
+  }
+#pragma unroll
+  for (int u = 0; u < kGroupPer; ++u) {
+    on[u] = on[u] && (what == 0 ? d.id[idx[u]] == d.gzone : d.ccnt[idx[u]] > 0);
+    any = any || on[u];
+  }
+  // (most chunks hold no particle of the zone or in contact)
+  if (__syncthreads_or(any)) {
+    for (int m = 0; m < nm; ++m) {
       double s[3] = {0, 0, 0};
-      for (int p = b + threadIdx.x; p < e; p += kGroupThreads) {
-        const int i = d.gidx[p];
-        if (d.ccnt[i] <= 0) continue;
-        const double4 f = d.gcf[(long long)m * d.npad + i];
-        s[0] += f.x, s[1] += f.y, s[2] += f.z;
+#pragma unroll
+      for (int u = 0; u < kGroupPer; ++u) {
+        if (!on[u]) continue;
+        if (what == 0) {
+          const double4 a = d.acc[idx[u]];
+          const double w = d.vm[idx[u]].w;
+          s[0] += w * a.x, s[1] += w * a.y, s[2] += w * a.z;
+        } else {
+          const double4 f = d.gcf[(long long)m * d.npad + idx[u]];
+          s[0] += f.x, s[1] += f.y, s[2] += f.z;
+        }
       }
       for (int k = 0; k < 3; ++k) {
-        const double r = block_reduce<0>(s[k], sh);
-        if (threadIdx.x == 0) d.gc_hist[(slot * kMaxMesh + m) * 3 + k] = r;
+        const double r = wave_sum(s[k]);
+        if ((tid & 63) == 0) sh[tid >> 6][3 * m + k] = r;
       }
     }
+  } else if (tid < 3 * nm) {
+    for (int w = 0; w < kGroupThreads / 64; ++w) sh[w][tid] = 0.0;
   }
+  __syncthreads();
+  const int nch = d.gnch[g];
+  if (tid < 3 * nm) {
+    double r = sh[0][tid];
+    for (int w = 1; w < kGroupThreads / 64; ++w) r += sh[w][tid];
+    put_agent(&d.gpart[(long long)blockIdx.x * kMaxMesh * 3 + tid], r);
+  }
+  stores_done();
+  __syncthreads();
+  if (tid == 0) last = atomicAdd(&d.gticket[g], 1) == nch - 1;
+  __syncthreads();
+  if (!last) return;
+  if (tid < 3 * nm) {
+    double r = 0.0;
+#pragma unroll 8
+    for (int c = 0; c < nch; ++c)
+      r += get_agent(&d.gpart[(long long)(ch.w + c) * kMaxMesh * 3 + tid]);
+    const long long slot = (d.flags->step % d.ghist_cap) * d.ngroups + g;
+    if (what == 0) d.gr_hist[slot * 3 + tid] = r;
+    else d.gc_hist[slot * kMaxMesh * 3 + tid] = r;
+  }
+  if (tid == 0) d.gticket[g] = 0;
 }
 
 void launch_group_sums(const Dev &d, hipStream_t st, int what) {
-  if (d.ngroups > 0) k_group_sums<<<d.ngroups, kGroupThreads, 0, st>>>(d, what);
+  if (d.ngroups > 0) k_group_sums<<<d.ngchunks, kGroupThreads, 0, st>>>(d, what);
 }
 
 // the drift of the rigid particles (the reference's loop covers them)
