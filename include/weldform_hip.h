@@ -149,7 +149,7 @@ typedef struct wf_config {
   int32_t device;           /* HIP device ordinal                              */
   int32_t no_graphs;        /* 1: launch kernels one by one instead of replaying
                                a captured HIP graph per step                  */
-  int32_t stage_max;        /* WF_MIXED: neighbours of each 128-particle tile are
+  int32_t stage_max;        /* neighbours of each 128-particle tile are
                                staged in LDS when the tile's neighbourhood has
                                at most this many particles (0: 896, the most;
                                -1: never, gather from HBM).  Results do not

@@ -429,6 +429,21 @@ DevMat to_dev(const wf_material &m) {
   return d;
 }
 
+// FP64: the passes from LDS take their smoothing length from the particle
+// itself, so every material's must be uniform; one or two lanes per particle
+// (asked for) leave too few wavefronts beside 60-120 KB of LDS per block and
+// gather from HBM
+void choose_f64(Ctx *c) {
+  std::vector<double> hm(kMaxMat, -1.0);
+  bool uni = true;
+  for (int64_t i = 0; i < c->n; ++i) {
+    double &r = hm[c->hi[WF_I_MATERIAL][i]];
+    if (r < 0) r = c->hf[WF_F_H][i];
+    else if (r != c->hf[WF_F_H][i]) uni = false;
+  }
+  c->d.lds64 = !c->d.mixed && uni && (c->cfg.lanes == 0 || c->cfg.lanes == kLanesLds64);
+}
+
 void allocate(Ctx *c) {
   Dev &d = c->d;
   const size_t np = (size_t)c->npad;
@@ -597,12 +612,11 @@ void allocate(Ctx *c) {
     for (size_t k = 0; k < 3 * np; ++k) eye[k] = 1.0;
     dput(c, d.gcm, eye);
   }
-  if (d.mixed) {
-    // stage_cnt = -1 marks a tile that gathers from HBM
-    d.stage_cnt = c->alloc<int>((size_t)d.ntiles);
-    HIPCHK(hipMemsetAsync(d.stage_cnt, 0xff, sizeof(int) * (size_t)d.ntiles, c->st));
-  }
-  if (d.mixed && c->cfg.stage_max >= 0) {
+  // stage_cnt = -1 marks a tile that gathers from HBM
+  d.stage_cnt = c->alloc<int>((size_t)d.ntiles);
+  HIPCHK(hipMemsetAsync(d.stage_cnt, 0xff, sizeof(int) * (size_t)d.ntiles, c->st));
+  choose_f64(c);
+  if (c->cfg.stage_max >= 0 && (d.mixed || d.lds64)) {
     d.stage_max = c->cfg.stage_max == 0 ? kStageMax : c->cfg.stage_max;
     d.stage = c->alloc<int>((size_t)d.ntiles * kStageMax);
     d.nbrl = c->alloc<uint16_t>((size_t)nb_rows(c->cfg.max_nb) * np);
@@ -1344,6 +1358,9 @@ int wf_set_field(void *ctx, int32_t field, const double *h) {
       case WF_F_H:
         put_d4(c, d.xh[0], h, 3, 1, 1);
         put_d4(c, d.xh[1], h, 3, 1, 1);
+        // the captured steps hold the pass the old lengths chose
+        choose_f64(c);
+        c->drop_graphs();
         break;
       case WF_F_V:
         put_d4(c, d.vm, h, 0, 3, 3);

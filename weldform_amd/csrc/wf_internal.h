@@ -16,7 +16,7 @@
 //           reads entries 4g..4g+3 as one int4 and the wave's load is one
 //           coalesced 1 KiB run
 //   stage   int32 [ntiles][kStageMax], nbrl uint16 [max_nb][npad]: the LDS
-//           staging lists of the mixed-precision pair passes
+//           staging lists of the pair passes that read from LDS
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -27,7 +27,7 @@ namespace wf {
 
 constexpr int kBlock = 128;
 constexpr int kScanChunk = 1024;  // cells per block of the counting sort's cell-start scan
-// LDS staging of the mixed-precision pair passes: a tile is one block of
+// LDS staging of the pair passes: a tile is one block of
 // kBlock consecutive particles; its staged set (the tile's particles and all
 // their neighbours, sorted by index) holds at most kStageMax particles.
 // 896 keeps 99.7 % of the tiles of a cubic lattice with 2h = 2.4 dx staged
@@ -41,7 +41,8 @@ constexpr int kStagePow2 = 1024;  // the power of two >= kStageMax the set sort 
 constexpr int kNbBatch = 8;
 constexpr int kMaxLanes = 4;     // threads per particle in a pair pass
 constexpr int kLanesMixed = 2;   // defaults (tuned on MI355X)
-constexpr int kLanesFP64 = 2;
+constexpr int kLanesFP64 = 2;    // the FP64 passes' HBM gathers
+constexpr int kLanesLds64 = 4;   // the FP64 passes from LDS
 __host__ __device__ inline long long nb_slot(long long npad, int k, long long i) {
   return ((long long)(k >> 2) * npad + i) * 4 + (k & 3);
 }
@@ -236,12 +237,13 @@ struct Dev {
   int *rcell, *rcount, *rstart, *rsorted;
   int *rrank, *rloc, *rtot, *roff;  // the rigid grid's counting sort, as above
   int *nnb, *nbr;
-  // LDS staging (mixed precision): per tile the sorted staged particle list
+  // LDS staging: per tile the sorted staged particle list
   // stage[t][0..stage_cnt[t]) (stage_cnt = -1: tile gathers from HBM), each
   // neighbour entry as a position in that list (nbrl, same layout as nbr)
   // and each particle's own position (selfl)
   int stage_max, ntiles;
-  int lanes_mx, lanes_f64;     // threads per particle in the pair passes
+  int lanes_mx, lanes_f64;     // threads per particle in the pair passes (FP64: the HBM gathers)
+  int lds64;                   // the FP64 passes read from LDS (kLanesLds64 threads per particle)
   int auto_ts;                 // bit 0 velocity, bit 1 acceleration criterion
   int ti_on;                   // some material has TI > 0
   int beta_on;                 // some material has a quadratic viscosity term (beta != 0)

@@ -12,6 +12,8 @@
 #include <float.h>
 #include <math.h>
 
+#include <type_traits>
+
 #include "wf_device.h"
 
 namespace wf {
@@ -937,6 +939,12 @@ void launch_neighbours(const Dev &d, hipStream_t st, int cur) {
 // ---------------------------------------------------------------------------
 // pass 1: acceleration (CalcAccel + AccelReduction, GradientType 0, TI = 0)
 
+// P / rho^2 with the equation of state's P
+__device__ inline double pr_of(double rho, double P0, double cs2, double rho0) {
+  const double ir = rcp_t(rho);
+  return (P0 + cs2 * (rho - rho0)) * ir * ir;
+}
+
 // Where a pass reads neighbour j: straight from HBM (Src<MX>, row of global
 // indices in nbr) or from the tile's LDS copy (row of staged positions in
 // nbrl).  Both give the same values, so results do not depend on staging.
@@ -970,17 +978,14 @@ struct HbmJ {
       else t[k] = d.tir[(long long)k * d.npad + j];
     }
   }
-  // P_j / rho_j^2 of the kinetic-energy pair term
-  __device__ R pr(int j, R rhoj, R P0, R cs2, R rho0) const {
-    if constexpr (MX) {
-      return d.prf[j];
-    } else {
-      const R irj = rcp_t(rhoj);
-      return (P0 + cs2 * (rhoj - rho0)) * irj * irj;
-    }
-  }
-  __device__ bool lower(int i, int j) const { return i < j; }
+  // m_j / rho_j and, with damage, the damage of particle j (FP64 passes)
+  __device__ R vol(int j) const { return S::vol(d, buf, j, R4{}); }
+  __device__ R dam(int j) const { return d.damD[j]; }
+  // P_j / rho_j^2 of the kinetic-energy pair term (FP64 passes)
+  __device__ R pr(int j, R P0, R cs2, R rho0) const { return pr_of(d.rho[buf][j], P0, cs2, rho0); }
+  __device__ bool lower(int j) const { return i < j; }
 };
+
 // Calls f(j) for the entries of a neighbour row of cnt entries that belong
 // to lane `sub` of the particle's `lanes` lanes: batches of kNbBatch entries
 // sub, sub + lanes, sub + 2 lanes, ... in row order, each batch's indices
@@ -1170,7 +1175,7 @@ __device__ inline void accel_lane(const Dev &d, int cur, int i, const G &g, int 
       if constexpr (!MX) {
         // damage weight of the pair (Source/InteractionAlt.cpp:54-60)
         if (d.damage) {
-          const R df = dam_weight(d.damD[i], d.damD[j]);
+          const R df = dam_weight(d.damD[i], g.dam(j));
           w = df > (R)0 ? (df * vj.w) * GK : (R)0;
         }
       }
@@ -1233,15 +1238,14 @@ __device__ inline int entry(const G &c, int u) {
 // groups beyond a row's end that the prefetch touches (at most 2 LANES + 1)
 // lie inside the allocation (nb_rows keeps kRowSpare spare entries) and are
 // never used.
+// a, b: the lane's first two groups (rows.group(2 sub) and the next), which
+// the kernels load before they stage the tile.
 template <int LANES, class Rows, class F>
 __device__ inline void walk_groups(const Rows &rows, int cnt, int sub, const typename Rows::G &self,
-                                   F &&group_fn) {
+                                   typename Rows::G a, typename Rows::G b, F &&group_fn) {
   static_assert(4 * (2 * LANES + 2) <= kRowSpare, "prefetch stays in the row allocation");
   const int ng = (cnt + 3) >> 2;
-  int g = 2 * sub;
-  typename Rows::G a = rows.group(g);
-  typename Rows::G b = rows.group(g + 1);
-  for (; g < ng; g += 2 * LANES) {
+  for (int g = 2 * sub; g < ng; g += 2 * LANES) {
     const typename Rows::G a2 = rows.group(g + 2 * LANES);
     const typename Rows::G b2 = rows.group(g + 2 * LANES + 1);
     // compiler-only barrier: the prefetch stays issued here (it may not be
@@ -1280,6 +1284,307 @@ __device__ inline float gk_f(float r2, const GkF &k) {
   const float t = fmaxf(2.0f - q, 0.0f);
   const float gout = (t * t) * (ri * k.gout);
   return q < 1.0f ? gin : gout;
+}
+
+// ---------------------------------------------------------------------------
+// FP64 pair passes from the tile's LDS copy, for contexts whose smoothing
+// length is uniform within each material (h_uni; the HBM gathers further down
+// cover the others).  The same rows, walk and branch-free pair arithmetic as
+// the mixed passes, in double.  LANES threads per particle; a tile that is
+// not staged reads the same records from HBM, in the same order.
+//
+// The HBM gathers are bound by the L1 and L2 traffic of 128 (acceleration),
+// 72 and 80 bytes per neighbour; the LDS copy is read from HBM once per tile
+// (~730 records for 128 particles), which leaves FP64 issue and LDS reads (112
+// bytes per pair in the acceleration) as the bounds.  Acceleration, density,
+// rates per launch at 976k particles (54.6 neighbours): gathers 735, 426 and
+// 480 us, from LDS 318, 146 and 191 us; at 4.5k particles 21.8, 16.1 and
+// 20.7 against 10.6, 7.3 and 9.5 us.
+//
+// A compile-time option (GC, BETA, DAM) costs no registers where it is off:
+// a runtime `if (damage)` in the walk split it into blocks and spilled 489
+// registers.
+
+struct GkD {
+  double ih, gin_a, gin_b, gout;  // 1/h, 2.25 c5, -3 c5, -0.75 c5 h
+};
+__device__ inline GkD gk_consts64(double h, int dim) {
+  const KH<double> k = kern_h_t<double>(h, dim);
+  return GkD{k.ih, 2.25 * k.c5, -3.0 * k.c5, -0.75 * k.c5 * h};
+}
+// 1/x and 1/sqrt(x): the hardware estimate (relative error d < 2^-23) and one
+// third-order step, 1/x = y / (1 - e) = y (1 + e + e^2 + ...) with
+// e = 1 - x y, and the series of (1 - e)^(-1/2): errors d^3 and below, under
+// the rounding
+__device__ inline double rcp3(double x) {
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(y, fma(e, e, e), y);
+}
+__device__ inline double rsqrt3(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+// gk_f in double
+__device__ inline double gk_d(double r2, const GkD &k) {
+  const double ri = rsqrt3(fmax(r2, DBL_MIN));
+  const double q = (r2 * ri) * k.ih;
+  const double gin = fma(q, k.gin_a, k.gin_b);
+  const double t = fmax(2.0 - q, 0.0);
+  const double gout = (t * t) * (ri * k.gout);
+  return q < 1.0 ? gin : gout;
+}
+
+// A tile's records in LDS, as arrays of 16-byte pairs: 16-byte reads of
+// consecutive positions cover every bank (32-byte records would use half of
+// them per read).  (x, y), (z, w), (vx, vy), (vz, u) with w and u = rho and m
+// (acceleration) or m/rho and m (rates); density: (x, y), (z, m/rho),
+// (vx, vy) and vz alone.  The acceleration adds sigma / rho^2 as three pairs.
+constexpr int kRecAccel = 7, kRecRates = 4, kRecDens = 3;  // pairs per record
+enum { PASS_ACCEL, PASS_DENS, PASS_RATES };
+template <int PASS>
+struct RecLds64 {
+  const double2 *r;
+  const double *s;   // vz (density), P/rho^2 (rates)
+  const double *dm;  // damage
+  __device__ void x(int p, double &x, double &y, double &z, double &w) const {
+    const double2 a = r[p], b = r[kStageMax + p];
+    x = a.x, y = a.y, z = b.x, w = b.y;
+  }
+  __device__ void v(int p, double &x, double &y, double &z, double &u) const {
+    const double2 a = r[2 * kStageMax + p];
+    x = a.x, y = a.y;
+    if constexpr (PASS == PASS_DENS) {
+      z = s[p], u = 0.0;
+    } else {
+      const double2 b = r[3 * kStageMax + p];
+      z = b.x, u = b.y;
+    }
+  }
+  __device__ void t(int p, double (&t)[6]) const {
+    const double2 a = r[4 * kStageMax + p], b = r[5 * kStageMax + p], c = r[6 * kStageMax + p];
+    t[0] = a.x, t[1] = a.y, t[2] = b.x, t[3] = b.y, t[4] = c.x, t[5] = c.y;
+  }
+  __device__ double pr(int p) const { return s[p]; }
+  __device__ double dam(int p) const { return dm[p]; }
+};
+template <int PASS>
+struct RecHbm64 {
+  const Dev &d;
+  const int buf;
+  __device__ void x(int j, double &x, double &y, double &z, double &w) const {
+    const double4 a = d.xh[buf][j];
+    x = a.x, y = a.y, z = a.z;
+    if (PASS == PASS_ACCEL) w = d.srec[j].rho;
+    else w = rec_vol(d, buf, j, PASS == PASS_RATES);
+  }
+  __device__ void v(int j, double &x, double &y, double &z, double &u) const {
+    const double4 a = d.vm[j];
+    x = a.x, y = a.y, z = a.z, u = a.w;
+  }
+  __device__ void t(int j, double (&t)[6]) const {
+    const StressRec q = d.srec[j];
+    for (int k = 0; k < 6; ++k) t[k] = q.s[k] * q.irho2;
+  }
+  __device__ double pr(int j) const { return rec_pr(d, buf, j); }
+  __device__ double dam(int j) const { return d.damD[j]; }
+  // m / rho, rounded to float in the rates of the Locking sums
+  __device__ static double rec_vol(const Dev &d, int buf, int j, bool rates) {
+    const double w = d.vol[buf][j];
+    return rates && d.locking ? (double)(float)w : w;
+  }
+  // P / rho^2 of the equation of state (pairs form within one material, so
+  // j's own material is the pair's)
+  __device__ static double rec_pr(const Dev &d, int buf, int j) {
+    const DevMat &M = d.mats[d.mat[j]];
+    return pr_of(d.rho[buf][j], M.P0, M.Cs * M.Cs, M.ref_density);
+  }
+};
+// all NT threads copy tile t's staged set into LDS; a thread's indices are
+// loaded first, then its records, then the barrier
+template <int NT, int PASS>
+__device__ inline void stage64(const Dev &d, int buf, int t, int U, double2 *r, double *sc, double *dm) {
+  constexpr int R = (kStageMax + NT - 1) / NT;
+  const int *st = d.stage + (long long)t * kStageMax;
+  const RecHbm64<PASS> h{d, buf};
+  int j[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int p = (int)threadIdx.x + q * NT;
+    j[q] = p < U ? st[p] : -1;
+  }
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    if (j[q] < 0) continue;
+    const int p = (int)threadIdx.x + q * NT;
+    double x, y, z, w, vx, vy, vz, u;
+    h.x(j[q], x, y, z, w);
+    h.v(j[q], vx, vy, vz, u);
+    if constexpr (PASS == PASS_ACCEL) {
+      double s[6];
+      h.t(j[q], s);
+      r[4 * kStageMax + p] = make_double2(s[0], s[1]);
+      r[5 * kStageMax + p] = make_double2(s[2], s[3]);
+      r[6 * kStageMax + p] = make_double2(s[4], s[5]);
+    }
+    if constexpr (PASS == PASS_RATES) sc[p] = h.pr(j[q]);
+    r[p] = make_double2(x, y);
+    r[kStageMax + p] = make_double2(z, w);
+    r[2 * kStageMax + p] = make_double2(vx, vy);
+    if constexpr (PASS == PASS_DENS) sc[p] = vz;
+    else r[3 * kStageMax + p] = make_double2(vz, u);
+    if constexpr (PASS != PASS_RATES)
+      if (d.damage) dm[p] = h.dam(j[q]);
+  }
+  __syncthreads();
+}
+
+// CalcAccel + AccelReduction (Source/InteractionAlt.cpp:12-260), as
+// accel_mx_lane in double, with the damage weight of the pair (:54-60)
+template <bool GC, bool BETA, bool DAM, class Rows, class Rec>
+__device__ inline void accel64_lane(const Dev &d, int i, int sub, int cnt, const double4 &xi, const double4 &vi,
+                                    const StressRec &ri, const Rows &rows, typename Rows::G a0, typename Rows::G b0,
+                                    const Rec &rec, double (&acc)[3]) {
+  double ax = 0, ay = 0, az = 0, sx = 0, sy = 0, sz = 0;
+  double Li[6];
+  own_corr<GC>(d, i, Li);
+  const DevMat &M = d.mats[d.mat[i]];
+  const double h = xi.w, rhoi = ri.rho;
+  const GkD k = gk_consts64(h, d.dim);
+  const double h2c = 0.01 * h * h, acs = M.alpha * M.Cs, bh = 0.5 * M.beta, hh = 2.0 * h, hha = hh * acs;
+  const double Di = DAM ? d.damD[i] : 0.0;
+  walk_groups<kLanesLds64>(rows, cnt, sub, rows.self(), a0, b0, [&](const typename Rows::G &c) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int p = entry(c, u);
+      double x, y, z, rho, vx, vy, vz, m, T[6];
+      rec.x(p, x, y, z, rho);
+      rec.v(p, vx, vy, vz, m);
+      rec.t(p, T);
+      const double dx = xi.x - x, dy = xi.y - y, dz = xi.z - z;
+      const double r2 = dx * dx + dy * dy + dz * dz;
+      const double GK = gk_d(r2, k);
+      const double vdot = (vi.x - vx) * dx + (vi.y - vy) * dy + (vi.z - vz) * dz;
+      const double D = rhoi + rho;
+      const double rd = rcp3((r2 + h2c) * D);
+      double pv;
+      if constexpr (BETA) {
+        const double hv = (hh * vdot) * rd;
+        pv = hv * fma(bh, hv * D, acs);
+      } else {
+        pv = (hha * vdot) * rd;
+      }
+      const double pi = vdot < 0.0 ? pv : 0.0;
+      double w = m * GK;
+      if constexpr (DAM) {
+        const double df = dam_weight(Di, rec.dam(p));
+        w = df > 0.0 ? (df * m) * GK : 0.0;
+      }
+      double ex, ey, ez;
+      corr_dir<GC>(Li, dx, dy, dz, ex, ey, ez);
+      ax = fma(w, fma(T[XX], ex, fma(T[XY], ey, fma(T[XZ], ez, pi * ex))), ax);
+      ay = fma(w, fma(T[XY], ex, fma(T[YY], ey, fma(T[YZ], ez, pi * ey))), ay);
+      az = fma(w, fma(T[XZ], ex, fma(T[YZ], ey, fma(T[ZZ], ez, pi * ez))), az);
+      sx = fma(w, ex, sx);
+      sy = fma(w, ey, sy);
+      sz = fma(w, ez, sz);
+      // at most two entries' records in registers
+      if (u & 1) __builtin_amdgcn_sched_barrier(0);
+    }
+  });
+  double t[6];
+  for (int q = 0; q < 6; ++q) t[q] = ri.s[q] * ri.irho2;
+  acc[0] = ax + (t[XX] * sx + t[XY] * sy + t[XZ] * sz);
+  acc[1] = ay + (t[XY] * sx + t[YY] * sy + t[YZ] * sz);
+  acc[2] = az + (t[XZ] * sx + t[YZ] * sy + t[ZZ] * sz);
+}
+
+// CalcDensInc + DensReduction (Source/InteractionAlt.cpp:483-640) with the
+// damage weight (:558-572)
+template <bool GC, bool DAM, class Rows, class Rec>
+__device__ inline double dens64_lane(const Dev &d, int i, int sub, int cnt, const double4 &xi, const double4 &vi,
+                                     const Rows &rows, typename Rows::G a0, typename Rows::G b0, const Rec &rec) {
+  double s = 0;
+  double Li[6];
+  own_corr<GC>(d, i, Li);
+  const GkD k = gk_consts64(xi.w, d.dim);
+  const double Di = DAM ? d.damD[i] : 0.0;
+  walk_groups<kLanesLds64>(rows, cnt, sub, rows.self(), a0, b0, [&](const typename Rows::G &c) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int p = entry(c, u);
+      double x, y, z, vol, vx, vy, vz, unused;
+      rec.x(p, x, y, z, vol);
+      rec.v(p, vx, vy, vz, unused);
+      const double dx = xi.x - x, dy = xi.y - y, dz = xi.z - z;
+      const double GK = gk_d(dx * dx + dy * dy + dz * dz, k);
+      double ex, ey, ez;
+      corr_dir<GC>(Li, dx, dy, dz, ex, ey, ez);
+      const double t = (vi.x - vx) * ex + (vi.y - vy) * ey + (vi.z - vz) * ez;
+      if constexpr (DAM) {
+        const double df = dam_weight(Di, rec.dam(p));
+        vol = df > 0.0 ? df * vol : 0.0;
+      }
+      s = fma(vol * GK, t, s);
+      if (u & 1) __builtin_amdgcn_sched_barrier(0);
+    }
+  });
+  return s;
+}
+
+// CalcRateTensors + RateTensorsReduction with the kinetic-energy pair term,
+// as rates_mx_lane in double; own is the particle's entry in its own row
+// (staged position or index)
+template <bool GC, class Rows, class Rec>
+__device__ inline void rates64_lane(const Dev &d, int i, int own, int sub, int cnt, const double4 &xi, const double4 &vi,
+                                    double pri, const Rows &rows, typename Rows::G a0, typename Rows::G b0,
+                                    const Rec &rec, double (&v)[10]) {
+  double dxx = 0, dyy = 0, dzz = 0, pxy = 0, qxy = 0, pxz = 0, qxz = 0, pyz = 0, qyz = 0, ek = 0;
+  double Li[6];
+  own_corr<GC>(d, i, Li);
+  const double mneg = -vi.w;
+  const GkD k = gk_consts64(xi.w, d.dim);
+  walk_groups<kLanesLds64>(rows, cnt, sub, rows.self(), a0, b0, [&](const typename Rows::G &c) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int p = entry(c, u);
+      double x, y, z, vol, ux, uy, uz, m;
+      rec.x(p, x, y, z, vol);
+      rec.v(p, ux, uy, uz, m);
+      const double pr = rec.pr(p);
+      const double dx = xi.x - x, dy = xi.y - y, dz = xi.z - z;
+      const double GK = gk_d(dx * dx + dy * dy + dz * dz, k);
+      const double vx = vi.x - ux, vy = vi.y - uy, vz = vi.z - uz;
+      const double cj = vol * GK;
+      double ex, ey, ez;
+      corr_dir<GC>(Li, dx, dy, dz, ex, ey, ez);
+      const double a = cj * ex, b = cj * ey, g = cj * ez;
+      dxx = fma(vx, a, dxx);
+      dyy = fma(vy, b, dyy);
+      dzz = fma(vz, g, dzz);
+      pxy = fma(vx, b, pxy);
+      qxy = fma(vy, a, qxy);
+      pxz = fma(vx, g, pxz);
+      qxz = fma(vz, a, qxz);
+      pyz = fma(vy, g, pyz);
+      qyz = fma(vz, b, qyz);
+      // staged positions follow particle index order
+      const double ms = own < p ? m : mneg;
+      ek = fma(ms * (pri + pr), GK * (vx * dx + vy * dy + vz * dz), ek);
+      if (u & 1) __builtin_amdgcn_sched_barrier(0);
+    }
+  });
+  v[XX] = -dxx;
+  v[YY] = -dyy;
+  v[ZZ] = -dzz;
+  v[XY] = -0.5 * (pxy + qxy);
+  v[XZ] = -0.5 * (pxz + qxz);
+  v[YZ] = -0.5 * (pyz + qyz);
+  v[6] = -0.5 * (pxy - qxy);
+  v[7] = -0.5 * (pxz - qxz);
+  v[8] = -0.5 * (pyz - qyz);
+  v[9] = 0.5 * ek;
 }
 
 // acceleration records of neighbour j: X = (x, y, z, rho), V = (v, m),
@@ -1325,7 +1630,7 @@ __device__ inline void accel_mx_lane(const Dev &d, int cur, int i, int sub, cons
   const GkF k = gk_consts(h, d.dim);
   const float h2c = 0.01f * h * h, hh = 2.0f * h;
   const float acs = (float)(M.alpha * M.Cs), bh = 0.5f * (float)M.beta, hha = hh * acs;
-  walk_groups<LANES>(rows, d.nnb[i], sub, rows.self(), [&](const typename Rows::G &c) {
+  walk_groups<LANES>(rows, d.nnb[i], sub, rows.self(), rows.group(2 * sub), rows.group(2 * sub + 1), [&](const typename Rows::G &c) {
     float4 X[4], V[4], T[4];
     float2 T2[4];
 #pragma unroll
@@ -1388,6 +1693,38 @@ __global__ __launch_bounds__(kBlock *LANES) void k_accel_f64(Dev d, int cur) {
   // plane strain: the pair forces have no z part (Source/InteractionAlt.cpp:
   // 184; the corrected-gradient terms keep theirs)
   if (d.dim == 2 && !d.gc_on) a[2] = 0.0;
+  if (i < d.n && sub == 0) d.acc[i] = make_double4(a[0], a[1], a[2], 0.0);
+}
+
+// FP64, uniform h: 112 bytes of LDS per staged particle, one block per CU.
+// The particle's own values and first row words are loaded before the tile
+// is staged, so their latency and the staging's overlap.
+template <bool GC, bool BETA, bool DAM>
+__global__ __launch_bounds__(kBlock *kLanesLds64) void k_accel64(Dev d, int cur) {
+  __shared__ double2 rec[kRecAccel * kStageMax];
+  __shared__ double dm[DAM ? kStageMax : 1];
+  __shared__ double red[(kLanesLds64 - 1) * 3 * kBlock];
+  const int t = xcd_tile(blockIdx.x, gridDim.x), sub = threadIdx.x / kBlock;
+  const int i = t * kBlock + (int)(threadIdx.x % kBlock);
+  const int U = d.stage_cnt[t];
+  const bool on = i < d.n && d.group[i] >= 0;
+  const int cnt = on ? d.nnb[i] : 0;
+  const double4 xi = d.xh[cur][i], vi = d.vm[i];
+  const StressRec ri = d.srec[i];
+  double a[3] = {0, 0, 0};
+  if (U < 0) {
+    const HbmRows rows{reinterpret_cast<const int4 *>(d.nbr) + i, d.npad, i};
+    if (on)
+      accel64_lane<GC, BETA, DAM>(d, i, sub, cnt, xi, vi, ri, rows, rows.group(2 * sub), rows.group(2 * sub + 1),
+                                    RecHbm64<PASS_ACCEL>{d, cur}, a);
+  } else {
+    const LdsRows rows{reinterpret_cast<const ushort4 *>(d.nbrl) + i, d.npad, (int)d.selfl[i]};
+    const ushort4 a0 = rows.group(2 * sub), b0 = rows.group(2 * sub + 1);
+    stage64<kBlock * kLanesLds64, PASS_ACCEL>(d, cur, t, U, rec, nullptr, dm);
+    if (on) accel64_lane<GC, BETA, DAM>(d, i, sub, cnt, xi, vi, ri, rows, a0, b0, RecLds64<PASS_ACCEL>{rec, nullptr, dm}, a);
+  }
+  combine_lanes<kLanesLds64>(a, red);
+  if (d.dim == 2 && !d.gc_on) a[2] = 0.0;  // plane strain, as k_accel_f64
   if (i < d.n && sub == 0) d.acc[i] = make_double4(a[0], a[1], a[2], 0.0);
 }
 
@@ -1459,6 +1796,13 @@ __global__ __launch_bounds__(kBlock *LANES) void k_accel_mx_ti(Dev d, int cur) {
     case 2: KERNEL<2><<<nblk(d.n), kBlock * 2, 0, st>>>(__VA_ARGS__); break;  \
     default: KERNEL<4><<<nblk(d.n), kBlock * 4, 0, st>>>(__VA_ARGS__); break; \
   }
+// the FP64 passes from LDS, by gradient correction and the pass's own options
+// (compile-time, so that the row walk has no branch)
+template <class F>
+static void gc_switch(bool gc, F &&f) {
+  if (gc) f(std::true_type{});
+  else f(std::false_type{});
+}
 // the mixed-precision passes are also instantiated per gradient correction
 #define WF_LANES_GC_SWITCH(lanes, gc, KERNEL, ...)                   \
   if (gc) {                                                         \
@@ -1542,7 +1886,21 @@ void launch_accel(const Dev &d, hipStream_t st, int cur) {
     WF_LANES_GC_SWITCH(d.lanes_mx, d.gc_on, k_accel_mx_b, d, cur)
   } else if (d.mixed) {
     WF_LANES_GC_SWITCH(d.lanes_mx, d.gc_on, k_accel_mx_nb, d, cur)
+  } else if (d.lds64 && !d.ti_on) {
+    gc_switch(d.gc_on, [&](auto gc) {
+      constexpr bool GC = decltype(gc)::value;
+      const dim3 g(nblk(d.n)), b(kBlock * kLanesLds64);
+      if (d.damage) {
+        if (d.beta_on) k_accel64<GC, true, true><<<g, b, 0, st>>>(d, cur);
+        else k_accel64<GC, false, true><<<g, b, 0, st>>>(d, cur);
+      } else {
+        if (d.beta_on) k_accel64<GC, true, false><<<g, b, 0, st>>>(d, cur);
+        else k_accel64<GC, false, false><<<g, b, 0, st>>>(d, cur);
+      }
+    });
   } else {
+    // FP64 with the tensile-instability stress or smoothing lengths that
+    // differ within a material
     WF_LANES_SWITCH(d.lanes_f64, k_accel_f64, d, cur)
   }
 }
@@ -1726,37 +2084,30 @@ void launch_kick2(const Dev &d, hipStream_t st, double dt) { k_kick2<<<nblk(d.n)
 //  Source/SolverLeapfrog.cpp:280-301).  Reads x_n, v_{n+1/2}, m/rho_n and
 // writes rho_{n+1}, m/rho_{n+1}, x_{n+1} into the other buffer.
 
-template <bool MX, bool GC, class G>
-__device__ inline typename Src<MX>::R dens_lane(const Dev &d, int cur, int i, const G &g, int sub, int lanes) {
-  using S = Src<MX>;
-  using R = typename S::R;
-  R s = 0;
+template <bool GC, class G>
+__device__ inline double dens_lane(const Dev &d, int cur, int i, const G &g, int sub, int lanes) {
+  using S = Src<false>;
+  double s = 0;
   if (d.group[i] >= 0) {
-    R Li[6];
+    double Li[6];
     own_corr<GC>(d, i, Li);
-    const auto xi = S::x(d, cur, i);
-    const auto vi = S::v(d, i);
-    const KH<R> ki = kern_h_t<R>(S::h_own(d, cur, i, xi), d.dim);
+    const double4 xi = S::x(d, cur, i), vi = S::v(d, i);
+    const KH<double> ki = kern_h_t<double>(xi.w, d.dim);
     for_each_nb(g, d.nnb[i], sub, lanes, [&](int j) {
-      const auto xj = g.x(j);
-      const auto vj = g.v(j);
-      const R volj = MX ? (R)xj.w : S::vol(d, cur, j, xj);
-      const R dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-      const R GK = gk_t<R>(dx * dx + dy * dy + dz * dz, S::kh(ki, xi, xj));
-      R ex, ey, ez;
+      const double4 xj = g.x(j), vj = g.v(j);
+      const double volj = g.vol(j);
+      const double dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+      const double GK = gk_t<double>(dx * dx + dy * dy + dz * dz, S::kh(ki, xi, xj));
+      double ex, ey, ez;
       corr_dir<GC>(Li, dx, dy, dz, ex, ey, ez);
-      if constexpr (MX) {
-        s += (volj * GK) * ((vi.x - vj.x) * ex + (vi.y - vj.y) * ey + (vi.z - vj.z) * ez);
-      } else {
-        const R t = (vi.x - vj.x) * (GK * ex) + (vi.y - vj.y) * (GK * ey) + (vi.z - vj.z) * (GK * ez);
-        R wv = volj;
-        // damage weight of the pair (Source/InteractionAlt.cpp:558-572)
-        if (d.damage) {
-          const R df = dam_weight(d.damD[i], d.damD[j]);
-          wv = df > (R)0 ? df * volj : (R)0;
-        }
-        s += wv * t;
+      const double t = (vi.x - vj.x) * (GK * ex) + (vi.y - vj.y) * (GK * ey) + (vi.z - vj.z) * (GK * ez);
+      double wv = volj;
+      // damage weight of the pair (Source/InteractionAlt.cpp:558-572)
+      if (d.damage) {
+        const double df = dam_weight(d.damD[i], g.dam(j));
+        wv = df > 0.0 ? df * volj : 0.0;
       }
+      s += wv * t;
     });
   }
   return s;
@@ -1810,10 +2161,40 @@ __global__ __launch_bounds__(kBlock *LANES) void k_dens_f64(Dev d, int cur, doub
   double s[1] = {0};
   if (i < d.n) {
     const HbmJ<false> g{d, cur, i};
-    s[0] = d.gc_on ? dens_lane<false, true>(d, cur, i, g, sub, LANES) : dens_lane<false, false>(d, cur, i, g, sub, LANES);
+    s[0] = d.gc_on ? dens_lane<true>(d, cur, i, g, sub, LANES) : dens_lane<false>(d, cur, i, g, sub, LANES);
   }
   combine_lanes<LANES>(s, red);
   if (i < d.n && sub == 0) dens_update<false>(d, cur, i, s[0], dt, do_update, dens_own(d, cur, i));
+}
+
+// FP64, uniform h: 56 bytes of LDS per staged particle, three blocks per CU
+// (two with damage)
+template <bool GC, bool DAM>
+__global__ __launch_bounds__(kBlock *kLanesLds64) void k_dens64(Dev d, int cur, double dt, int do_update) {
+  __shared__ double2 rec[kRecDens * kStageMax];
+  __shared__ double sc[kStageMax];
+  __shared__ double dm[DAM ? kStageMax : 1];
+  __shared__ double red[(kLanesLds64 - 1) * kBlock];
+  const int t = xcd_tile(blockIdx.x, gridDim.x), sub = threadIdx.x / kBlock;
+  const int i = t * kBlock + (int)(threadIdx.x % kBlock);
+  const int U = d.stage_cnt[t];
+  const bool on = i < d.n && d.group[i] >= 0;
+  const int cnt = on ? d.nnb[i] : 0;
+  const double4 xi = d.xh[cur][i], vi = d.vm[i];
+  double s[1] = {0};
+  if (U < 0) {
+    const HbmRows rows{reinterpret_cast<const int4 *>(d.nbr) + i, d.npad, i};
+    if (on)
+      s[0] = dens64_lane<GC, DAM>(d, i, sub, cnt, xi, vi, rows, rows.group(2 * sub), rows.group(2 * sub + 1),
+                                    RecHbm64<PASS_DENS>{d, cur});
+  } else {
+    const LdsRows rows{reinterpret_cast<const ushort4 *>(d.nbrl) + i, d.npad, (int)d.selfl[i]};
+    const ushort4 a0 = rows.group(2 * sub), b0 = rows.group(2 * sub + 1);
+    stage64<kBlock * kLanesLds64, PASS_DENS>(d, cur, t, U, rec, sc, dm);
+    if (on) s[0] = dens64_lane<GC, DAM>(d, i, sub, cnt, xi, vi, rows, a0, b0, RecLds64<PASS_DENS>{rec, sc, dm});
+  }
+  combine_lanes<kLanesLds64>(s, red);
+  if (i < d.n && sub == 0) dens_update<false>(d, cur, i, s[0], dt, do_update, DensOwn{d.rho[cur][i], xi, vi, d.disp[i]});
 }
 
 // records of the density and rate passes: X = (x, y, z, m/rho), V = (v, m)
@@ -1846,7 +2227,7 @@ __device__ inline float dens_mx_lane(const Dev &d, int cur, int i, int sub, cons
   own_corr<GC>(d, i, Li);
   const float4 xi = d.xhf[cur][i], vi = d.vmf[i];
   const GkF k = gk_consts((float)d.xh[cur][i].w, d.dim);
-  walk_groups<LANES>(rows, d.nnb[i], sub, rows.self(), [&](const typename Rows::G &c) {
+  walk_groups<LANES>(rows, d.nnb[i], sub, rows.self(), rows.group(2 * sub), rows.group(2 * sub + 1), [&](const typename Rows::G &c) {
     float4 X[4], V[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) rec.load(entry(c, u), X[u], V[u]);
@@ -1894,7 +2275,16 @@ void launch_dens_drift(const Dev &d, hipStream_t st, int cur, double dt, int do_
   if (d.mixed) {
     WF_LANES_GC_SWITCH(d.lanes_mx, d.gc_on, k_dens_mx, d, cur, dt, do_update)
   } else {
-    WF_LANES_SWITCH(d.lanes_f64, k_dens_f64, d, cur, dt, do_update)
+    if (d.lds64) {
+      gc_switch(d.gc_on, [&](auto gc) {
+        constexpr bool GC = decltype(gc)::value;
+        const dim3 g(nblk(d.n)), b(kBlock * kLanesLds64);
+        if (d.damage) k_dens64<GC, true><<<g, b, 0, st>>>(d, cur, dt, do_update);
+        else k_dens64<GC, false><<<g, b, 0, st>>>(d, cur, dt, do_update);
+      });
+    } else {
+      WF_LANES_SWITCH(d.lanes_f64, k_dens_f64, d, cur, dt, do_update)
+    }
   }
 }
 
@@ -1910,39 +2300,34 @@ void launch_dens_drift(const Dev &d, hipStream_t st, int cur, double dt, int do_
 
 // one particle's rate-tensor gather: v[0..5] strain rate, v[6..8] rotation
 // rate (w01, w02, w12), v[9] the kinetic-energy pair sum
-// LK: the Locking sums' weight, m_j / rho_j rounded to float (the FP32
-// path's weight already is)
-template <bool MX, bool GC, bool LK, class G>
-__device__ inline void rates_lane(const Dev &d, int buf, int i, const G &g, int sub, int lanes,
-                                  typename Src<MX>::R (&v)[10]) {
-  using Sr = Src<MX>;
-  using R = typename Sr::R;
-  R sr[6] = {0, 0, 0, 0, 0, 0}, w[3] = {0, 0, 0};
-  R ekin = 0;
+// LK: the Locking sums' weight, m_j / rho_j rounded to float
+template <bool GC, bool LK, class G>
+__device__ inline void rates_lane(const Dev &d, int buf, int i, const G &g, int sub, int lanes, double (&v)[10]) {
+  using Sr = Src<false>;
+  double sr[6] = {0, 0, 0, 0, 0, 0}, w[3] = {0, 0, 0};
+  double ekin = 0;
   if (d.group[i] >= 0) {
-    R Li[6];
+    double Li[6];
     own_corr<GC>(d, i, Li);
     const DevMat &M = d.mats[d.mat[i]];
-    const auto xi = Sr::x(d, buf, i);
-    const auto vi = Sr::v(d, i);
-    const R P0 = (R)M.P0, cs2 = (R)(M.Cs * M.Cs), rho0 = (R)M.ref_density;
-    const R pri = g.pr(MX ? g.self() : i, MX ? (R)0 : Sr::rho(d, buf, i, xi, vi), P0, cs2, rho0);
-    const R mi = vi.w;
-    const KH<R> ki = kern_h_t<R>(Sr::h_own(d, buf, i, xi), d.dim);
+    const double4 xi = Sr::x(d, buf, i), vi = Sr::v(d, i);
+    const double P0 = M.P0, cs2 = M.Cs * M.Cs, rho0 = M.ref_density;
+    const double pri = g.pr(g.self(), P0, cs2, rho0);
+    const double mi = vi.w;
+    const KH<double> ki = kern_h_t<double>(xi.w, d.dim);
     for_each_nb(g, d.nnb[i], sub, lanes, [&](int j) {
-      const auto xj = g.x(j);
-      const auto vj = g.v(j);
-      R volj = MX ? (R)xj.w : Sr::vol(d, buf, j, xj);
-      if constexpr (LK && !MX) volj = (R)(float)volj;
-      const R dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-      const R GK = gk_t<R>(dx * dx + dy * dy + dz * dz, Sr::kh(ki, xi, xj));
-      const R vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
-      const R c = volj * ((R)-0.5 * GK);
-      R ex, ey, ez;
+      const double4 xj = g.x(j), vj = g.v(j);
+      double volj = g.vol(j);
+      if constexpr (LK) volj = (double)(float)volj;
+      const double dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+      const double GK = gk_t<double>(dx * dx + dy * dy + dz * dz, Sr::kh(ki, xi, xj));
+      const double vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
+      const double c = volj * (-0.5 * GK);
+      double ex, ey, ez;
       corr_dir<GC>(Li, dx, dy, dz, ex, ey, ez);
-      sr[XX] += c * ((R)2 * vx * ex);
-      sr[YY] += c * ((R)2 * vy * ey);
-      sr[ZZ] += c * ((R)2 * vz * ez);
+      sr[XX] += c * (2.0 * vx * ex);
+      sr[YY] += c * (2.0 * vy * ey);
+      sr[ZZ] += c * (2.0 * vz * ez);
       sr[XY] += c * (vx * ey + vy * ex);
       sr[XZ] += c * (vx * ez + vz * ex);
       sr[YZ] += c * (vy * ez + vz * ey);
@@ -1951,10 +2336,10 @@ __device__ inline void rates_lane(const Dev &d, int buf, int i, const G &g, int 
       w[2] += c * (vy * ez - vz * ey);
       // kinetic-energy pair term (Source/Domain.cpp:1776-1792): the pair
       // is oriented lower-index first; its sum over particles vanishes
-      const R prj = g.pr(j, MX ? (R)0 : Sr::rho(d, buf, j, xj, vj), P0, cs2, rho0);
-      const bool lo = g.lower(i, j);
-      const R msec = lo ? vj.w : mi;
-      const R term = (R)0.5 * msec * (pri + prj) * (vx * (GK * dx) + vy * (GK * dy) + vz * (GK * dz));
+      const double prj = g.pr(j, P0, cs2, rho0);
+      const bool lo = g.lower(j);
+      const double msec = lo ? vj.w : mi;
+      const double term = 0.5 * msec * (pri + prj) * (vx * (GK * dx) + vy * (GK * dy) + vz * (GK * dz));
       ekin += lo ? term : -term;
     });
   }
@@ -1981,14 +2366,48 @@ __global__ __launch_bounds__(kBlock *LANES) void k_rates_f64(Dev d, int buf) {
   if (i < d.n) {
     const HbmJ<false> g{d, buf, i};
     if (d.gc_on) {
-      if (d.locking) rates_lane<false, true, true>(d, buf, i, g, sub, LANES, v);
-      else rates_lane<false, true, false>(d, buf, i, g, sub, LANES, v);
+      if (d.locking) rates_lane<true, true>(d, buf, i, g, sub, LANES, v);
+      else rates_lane<true, false>(d, buf, i, g, sub, LANES, v);
     } else {
-      if (d.locking) rates_lane<false, false, true>(d, buf, i, g, sub, LANES, v);
-      else rates_lane<false, false, false>(d, buf, i, g, sub, LANES, v);
+      if (d.locking) rates_lane<false, true>(d, buf, i, g, sub, LANES, v);
+      else rates_lane<false, false>(d, buf, i, g, sub, LANES, v);
     }
   }
   combine_lanes<LANES>(v, red);
+  const double e_kin = (i < d.n && sub == 0) ? rates_store(d, i, v) : 0.0;
+  const double r1 = block_reduce<0>(e_kin, sh);
+  if (threadIdx.x == 0) part(d, P_KIN, blockIdx.x) = r1;
+}
+
+// FP64, uniform h: 72 bytes of LDS per staged particle, two blocks per CU;
+// the lanes' partial sums reuse the records' space
+template <bool GC>
+__global__ __launch_bounds__(kBlock *kLanesLds64) void k_rates64(Dev d, int buf) {
+  __shared__ double2 rec[kRecRates * kStageMax];
+  __shared__ double sc[kStageMax];
+  static_assert(2 * kRecRates * kStageMax >= (kLanesLds64 - 1) * 10 * kBlock, "the partial sums fit the records' space");
+  __shared__ double sh[kBlock * kLanesLds64 / 64];
+  const int t = xcd_tile(blockIdx.x, gridDim.x), sub = threadIdx.x / kBlock;
+  const int i = t * kBlock + (int)(threadIdx.x % kBlock);
+  const int U = d.stage_cnt[t];
+  const bool on = i < d.n && d.group[i] >= 0;
+  const int cnt = on ? d.nnb[i] : 0;
+  const double4 xi = d.xh[buf][i], vi = d.vm[i];
+  double v[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  if (U < 0) {
+    const HbmRows rows{reinterpret_cast<const int4 *>(d.nbr) + i, d.npad, i};
+    if (on)
+      rates64_lane<GC>(d, i, i, sub, cnt, xi, vi, RecHbm64<PASS_RATES>::rec_pr(d, buf, i), rows,
+                              rows.group(2 * sub), rows.group(2 * sub + 1), RecHbm64<PASS_RATES>{d, buf}, v);
+  } else {
+    const LdsRows rows{reinterpret_cast<const ushort4 *>(d.nbrl) + i, d.npad, (int)d.selfl[i]};
+    const ushort4 a0 = rows.group(2 * sub), b0 = rows.group(2 * sub + 1);
+    stage64<kBlock * kLanesLds64, PASS_RATES>(d, buf, t, U, rec, sc, nullptr);
+    const RecLds64<PASS_RATES> l{rec, sc, nullptr};
+    if (on) rates64_lane<GC>(d, i, rows.own, sub, cnt, xi, vi, l.pr(rows.own), rows, a0, b0, l, v);
+  }
+  __syncthreads();  // the records are read before the partial sums overwrite them
+  combine_lanes<kLanesLds64>(v, reinterpret_cast<double *>(rec));
   const double e_kin = (i < d.n && sub == 0) ? rates_store(d, i, v) : 0.0;
   const double r1 = block_reduce<0>(e_kin, sh);
   if (threadIdx.x == 0) part(d, P_KIN, blockIdx.x) = r1;
@@ -2013,7 +2432,7 @@ __device__ inline void rates_mx_lane(const Dev &d, int buf, int i, int own, int 
   const float4 xi = d.xhf[buf][i], vi = d.vmf[i];
   const float pri = d.prf[i], mneg = -vi.w;
   const GkF k = gk_consts((float)d.xh[buf][i].w, d.dim);
-  walk_groups<LANES>(rows, d.nnb[i], sub, rows.self(), [&](const typename Rows::G &c) {
+  walk_groups<LANES>(rows, d.nnb[i], sub, rows.self(), rows.group(2 * sub), rows.group(2 * sub + 1), [&](const typename Rows::G &c) {
     float4 X[4], V[4];
     float P[4];
     int l[4];
@@ -2235,7 +2654,13 @@ void launch_rates(const Dev &d, hipStream_t st, int buf) {
   if (d.mixed) {
     WF_LANES_GC_SWITCH(d.lanes_mx, d.gc_on, k_rates_mx, d, buf)
   } else {
-    WF_LANES_SWITCH(d.lanes_f64, k_rates_f64, d, buf)
+    if (d.lds64) {
+      gc_switch(d.gc_on, [&](auto gc) {
+        k_rates64<decltype(gc)::value><<<nblk(d.n), kBlock * kLanesLds64, 0, st>>>(d, buf);
+      });
+    } else {
+      WF_LANES_SWITCH(d.lanes_f64, k_rates_f64, d, buf)
+    }
   }
 }
 
