@@ -441,6 +441,7 @@ void choose_f64(Ctx *c) {
     if (r < 0) r = c->hf[WF_F_H][i];
     else if (r != c->hf[WF_F_H][i]) uni = false;
   }
+  c->d.h_uni = uni;
   c->d.lds64 = !c->d.mixed && uni && (c->cfg.lanes == 0 || c->cfg.lanes == kLanesLds64);
 }
 
@@ -496,6 +497,7 @@ void allocate(Ctx *c) {
   d.sinfo = c->alloc<int2>(np + 4);
   d.soff = c->alloc<int4>((size_t)d.sncells);
   d.sslice = c->alloc<unsigned char>(np);
+  if (d.thermal) d.tkey = c->alloc<long long>(np);
   d.hblk = c->alloc<unsigned>((size_t)d.nblocks);
   c->dmats = c->alloc<DevMat>(kMaxMat);
   d.mats = c->dmats;
@@ -1079,7 +1081,7 @@ void enqueue_step(Ctx *c, int scheme, int cur, const TapeHook *tp = nullptr, int
       launch_rates(d, c->st, nxt);
     }
     launch_stress(d, c->st, nxt, dt);
-    if (c->cfg.thermal_solver) launch_thermal(d, c->st, nxt, dt);
+    if (c->cfg.thermal_solver) launch_thermal(d, c->st, nxt);
     launch_finalize(d, c->st, dt, c->bc.nz);
     if (d.contact) launch_mesh_update(d, c->st, dt);
     if (tp) {

@@ -230,6 +230,9 @@ struct Dev {
   // cell's records are ordered by the quarter of the cell height they lie
   // in, then by index), and the cell's end
   int4 *soff;
+  // with the thermal solver: orders the two particles of a pair as the
+  // reference's pair list does (see thermal_key), set with `cell`
+  long long *tkey;
   unsigned char *sslice;  // each particle's z-slice in its search cell
   unsigned *hblk;         // per block of particles: the largest FP32 h (bits)
   // rigid (contact) particles binned in the same cells: counts, starts,
@@ -243,6 +246,7 @@ struct Dev {
   // and each particle's own position (selfl)
   int stage_max, ntiles;
   int lanes_mx, lanes_f64;     // threads per particle in the pair passes (FP64: the HBM gathers)
+  int h_uni;                   // every material's smoothing length is uniform
   int lds64;                   // the FP64 passes read from LDS (kLanesLds64 threads per particle)
   int auto_ts;                 // bit 0 velocity, bit 1 acceleration criterion
   int ti_on;                   // some material has TI > 0
@@ -380,7 +384,7 @@ void launch_kick2(const Dev &d, hipStream_t st, double dt);
 void launch_dens_drift(const Dev &d, hipStream_t st, int cur, double dt, int do_update);
 void launch_rates(const Dev &d, hipStream_t st, int buf);
 void launch_stress(const Dev &d, hipStream_t st, int buf, double dt);
-void launch_thermal(const Dev &d, hipStream_t st, int buf, double dt);
+void launch_thermal(const Dev &d, hipStream_t st, int buf);
 void launch_finalize(const Dev &d, hipStream_t st, double dt, int nz);
 void launch_max_pl(const Dev &d, hipStream_t st);
 void launch_shadows(const Dev &d, hipStream_t st, int cur);

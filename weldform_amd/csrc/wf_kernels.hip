@@ -135,6 +135,19 @@ __device__ inline int scell_of(const Dev &d, const double4 x) {
   return (cx * d.scellno[1] + cy) * d.scellno[2] + cz;
 }
 
+// The order of a pair's particles in the reference's list: "first" is the
+// particle whose cell the pair was found from (Source/Neighbour.cpp:418-477),
+// the higher index within one cell, else the particle whose half stencil
+// holds the other, i.e. with the cells' offset (dx, dy, dz) = cell_j - cell_i,
+// each -1, 0 or 1: dz = 1, or dz = 0 and dy = 1, or dz = dy = 0 and dx = 1.
+// That is the sign of dx + 3 dy + 9 dz, so one comparison of these keys
+// decides: i is first where key_j > key_i.
+__device__ inline long long thermal_key(const Dev &d, int c, int perm) {
+  const int nz = d.cellno[2], ny = d.cellno[1];
+  const int cz = c % nz, cy = (c / nz) % ny, cx = c / (nz * ny);
+  return ((long long)(cx + 3 * cy + 9 * cz) << 32) | (unsigned)(0x7fffffff - perm);
+}
+
 // threads 0..n-1: the SPH particles; n..n+nrig-1: the rigid particles.
 // The counts are zero on entry (allocation, then cleared by k_cell_sort
 // once a search has consumed them).
@@ -163,7 +176,9 @@ WF_KERNEL void k_cell_hist(Dev d, int cur) {
   if (i < d.n) {
     const double4 x = d.xh[cur][i];
     hb = __float_as_uint((float)x.w);
-    d.cell[i] = cell_of(d, x);
+    const int rc = cell_of(d, x);
+    d.cell[i] = rc;
+    if (d.thermal) d.tkey[i] = thermal_key(d, rc, d.perm[i]);
     c = scell_of(d, x);
     d.scell[i] = c;
     const int cz = c % d.scellno[2];
@@ -1401,13 +1416,12 @@ struct RecHbm64 {
     return pr_of(d.rho[buf][j], M.P0, M.Cs * M.Cs, M.ref_density);
   }
 };
-// all NT threads copy tile t's staged set into LDS; a thread's indices are
-// loaded first, then its records, then the barrier
-template <int NT, int PASS>
-__device__ inline void stage64(const Dev &d, int buf, int t, int U, double2 *r, double *sc, double *dm) {
+// all NT threads call put(p, j) for the entries of tile t's staged set (each
+// thread's indices are loaded first), then meet at a barrier
+template <int NT, class F>
+__device__ inline void stage_set(const Dev &d, int t, int U, F &&put) {
   constexpr int R = (kStageMax + NT - 1) / NT;
   const int *st = d.stage + (long long)t * kStageMax;
-  const RecHbm64<PASS> h{d, buf};
   int j[R];
 #pragma unroll
   for (int q = 0; q < R; ++q) {
@@ -1415,29 +1429,33 @@ __device__ inline void stage64(const Dev &d, int buf, int t, int U, double2 *r, 
     j[q] = p < U ? st[p] : -1;
   }
 #pragma unroll
-  for (int q = 0; q < R; ++q) {
-    if (j[q] < 0) continue;
-    const int p = (int)threadIdx.x + q * NT;
+  for (int q = 0; q < R; ++q)
+    if (j[q] >= 0) put((int)threadIdx.x + q * NT, j[q]);
+  __syncthreads();
+}
+template <int NT, int PASS>
+__device__ inline void stage64(const Dev &d, int buf, int t, int U, double2 *r, double *sc, double *dm) {
+  const RecHbm64<PASS> h{d, buf};
+  stage_set<NT>(d, t, U, [&](int p, int j) {
     double x, y, z, w, vx, vy, vz, u;
-    h.x(j[q], x, y, z, w);
-    h.v(j[q], vx, vy, vz, u);
+    h.x(j, x, y, z, w);
+    h.v(j, vx, vy, vz, u);
     if constexpr (PASS == PASS_ACCEL) {
       double s[6];
-      h.t(j[q], s);
+      h.t(j, s);
       r[4 * kStageMax + p] = make_double2(s[0], s[1]);
       r[5 * kStageMax + p] = make_double2(s[2], s[3]);
       r[6 * kStageMax + p] = make_double2(s[4], s[5]);
     }
-    if constexpr (PASS == PASS_RATES) sc[p] = h.pr(j[q]);
+    if constexpr (PASS == PASS_RATES) sc[p] = h.pr(j);
     r[p] = make_double2(x, y);
     r[kStageMax + p] = make_double2(z, w);
     r[2 * kStageMax + p] = make_double2(vx, vy);
     if constexpr (PASS == PASS_DENS) sc[p] = vz;
     else r[3 * kStageMax + p] = make_double2(vz, u);
     if constexpr (PASS != PASS_RATES)
-      if (d.damage) dm[p] = h.dam(j[q]);
-  }
-  __syncthreads();
+      if (d.damage) dm[p] = h.dam(j);
+  });
 }
 
 // CalcAccel + AccelReduction (Source/InteractionAlt.cpp:12-260), as
@@ -2675,88 +2693,175 @@ void launch_stress(const Dev &d, hipStream_t st, int buf, double dt) {
 // conduction (CalcTempInc, Source/Thermal.cpp:53-219) + convection
 // (CalcConvHeat, :339-389) + thermal expansion (Source/ThermalStuct.cpp:7-12)
 // The reference credits temp[first] += m and temp[second] -= m with m built
-// from the second particle's m/rho; "first" is the particle whose cell the
-// pair was found from (Source/Neighbour.cpp:418-477): the higher index
-// within one cell, else the particle whose half stencil holds the other.
+// from the second particle's m/rho (first, second: see thermal_key).  FP64 in
+// both precision modes.
+//
+// The gather kernel (one lane per particle; positions, T, m/rho, cells and
+// indices of each neighbour from HBM, the cells' order by integer divisions)
+// took 211 us at 370k particles, bound by the latency of its dependent loads.
+// From the tile's LDS copy (48 bytes per staged particle) 64 us with two lanes
+// and three blocks per CU, 79 us with four lanes (two blocks, register bound).
+// The gather remains for smoothing lengths that differ within a material.
 
-__device__ inline bool pair_first(int ci, int cj, int oi, int oj, int ny, int nz) {
-  if (ci == cj) return oi > oj;
-  const int zi = ci % nz, yi = (ci / nz) % ny, xi = ci / (nz * ny);
-  const int zj = cj % nz, yj = (cj / nz) % ny, xj = cj / (nz * ny);
-  const int dx = xj - xi, dy = yj - yi, dz = zj - zi;
-  return dz == 1 || (dz == 0 && dy == 1) || (dz == 0 && dy == 0 && dx == 1);
-}
-
-WF_KERNEL void k_thermal(Dev d, int buf, double dt) {
-  if (dt < 0) dt = d.flags->dt;
-  __shared__ double sh[kBlock / 64];
-  const int i = xcd_tile(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+// the particle's own side after the gather: convection, sources, dT/dt, the
+// thermal strain rate; returns the internal energy rate and the contact heat
+// totals' terms (Source/Thermal.cpp:194-210)
+__device__ inline double3 thermal_own(const Dev &d, int buf, int i, double temp) {
   const long long np = d.npad;
-  double e_int = 0.0, e_frw = 0.0, e_chc = 0.0;
-  if (i < d.n && d.group[i] >= 0) {
-    const DevMat &M = d.mats[d.mat[i]];
-    const double4 xi = d.xh[buf][i];
-    const double rho = d.rho[buf][i];
-    const double m = d.vm[i].w;
-    const double Ti = d.T[i];
-    const double voli = d.vol[buf][i];
-    if (d.thbc[i] == 1) {
-      // (m/rho)^(2/3), (m/rho)^(1/3) in plane strain (Source/Thermal.cpp:354-366)
-      const double dS2 = pow(m / rho, d.dim == 2 ? 1.0 / 3.0 : 2.0 / 3.0);
-      d.qconv[i] = rho * d.hconv[i] * dS2 * (d.tinf[i] - Ti) / m;
+  const DevMat &M = d.mats[d.mat[i]];
+  const double rho = d.rho[buf][i], m = d.vm[i].w, Ti = d.T[i], voli = d.vol[buf][i];
+  double qconv = d.qconv[i];
+  if (d.thbc[i] == 1) {
+    // (m/rho)^(2/3), (m/rho)^(1/3) in plane strain (Source/Thermal.cpp:354-366)
+    const double dS2 = pow(m / rho, d.dim == 2 ? 1.0 / 3.0 : 2.0 / 3.0);
+    qconv = rho * d.hconv[i] * dS2 * (d.tinf[i] - Ti) / m;
+    d.qconv[i] = qconv;
+  }
+  const double f = 1. / (rho * M.cp_T);
+  const double qc = d.heat_cond ? d.qcont[i] : 0.0;
+  double dTdt = f * (temp + qconv + d.qsrc[i] + d.qpl[i] * d.pl_frac + qc);
+  if (d.heat_fric) dTdt += f * d.qfric[i];
+  d.dTdt[i] = dTdt;
+  double3 e = make_double3(0.0, 0.0, 0.0);
+  if (d.qfric) {
+    e.y = d.qfric[i] * m / rho;
+    e.z = qc * m / rho;
+  }
+  double SR[6];
+  for (int k = 0; k < 6; ++k) SR[k] = d.sr[k * np + i];
+  const double ex = M.th_exp * dTdt;
+  for (int k = 0; k < 3; ++k) {
+    SR[k] += ex;
+    d.sr[k * np + i] = SR[k];
+  }
+  double S[6];
+  for (int k = 0; k < 6; ++k) S[k] = d.S[k * np + i];
+  e.x = voli * (S[XX] * SR[XX] + 2.0 * S[XY] * SR[XY] + 2.0 * S[XZ] * SR[XZ] + S[YY] * SR[YY] +
+                2.0 * S[YZ] * SR[YZ] + S[ZZ] * SR[ZZ]);
+  return e;
+}
+__device__ inline void thermal_sums(const Dev &d, const double3 &e, int t, double *sh) {
+  const double r0 = block_reduce<0>(e.x, sh);
+  if (threadIdx.x == 0) part(d, P_INT, t) = r0;
+  if (d.qfric) {
+    const double r1 = block_reduce<0>(e.y, sh);
+    const double r2 = block_reduce<0>(e.z, sh);
+    if (threadIdx.x == 0) {
+      part(d, P_FRW, t) = r1;
+      part(d, P_CHC, t) = r2;
     }
-    const double kk = 4. * (M.k_T * M.k_T) / (M.k_T + M.k_T);
-    const int ci = d.cell[i], oi = d.perm[i];
+  }
+}
+// the conductivity factor of a pair (both particles of one material)
+__device__ inline double pair_kk(const DevMat &M) { return 4. * (M.k_T * M.k_T) / (M.k_T + M.k_T); }
+
+WF_KERNEL void k_thermal(Dev d, int buf) {
+  __shared__ double sh[kBlock / 64];
+  const int t = xcd_tile(blockIdx.x, gridDim.x);
+  const int i = t * kBlock + threadIdx.x;
+  double3 e = make_double3(0.0, 0.0, 0.0);
+  if (i < d.n && d.group[i] >= 0) {
+    const double4 xi = d.xh[buf][i];
+    const double Ti = d.T[i], voli = d.vol[buf][i], kk = pair_kk(d.mats[d.mat[i]]);
+    const long long ki = d.tkey[i];
     double temp = 0.0;
-    const KernH ki = kern_h(xi.w, d.dim);
+    const KernH kh = kern_h(xi.w, d.dim);
     const int cnt = d.nnb[i];
     for (int k = 0; k < cnt; ++k) {
-      const int j = d.nbr[nb_slot(np, k, i)];
+      const int j = d.nbr[nb_slot(d.npad, k, i)];
       const double4 xj = d.xh[buf][j];
       const double dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
       const double r2 = dx * dx + dy * dy + dz * dz;
-      const double GK = grad_kernel_r2(r2, pair_h(ki, xi.w, xj.w));
-      const bool first = pair_first(ci, d.cell[j], oi, d.perm[j], d.cellno[1], d.cellno[2]);
-      const double vsec = first ? d.vol[buf][j] : voli;
+      const double GK = grad_kernel_r2(r2, pair_h(kh, xi.w, xj.w));
+      const double vsec = d.tkey[j] > ki ? d.vol[buf][j] : voli;
       // dot(x_ij, GK x_ij) / |x_ij|^2 = GK
       temp += vsec * kk * (Ti - d.T[j]) * GK;
     }
-    const double f = 1. / (rho * M.cp_T);
-    const double qc = d.heat_cond ? d.qcont[i] : 0.0;
-    double dTdt = f * (temp + d.qconv[i] + d.qsrc[i] + d.qpl[i] * d.pl_frac + qc);
-    if (d.heat_fric) dTdt += f * d.qfric[i];
-    d.dTdt[i] = dTdt;
-    if (d.qfric) {
-      // the contact heat totals (Source/Thermal.cpp:194-210)
-      e_frw = d.qfric[i] * m / rho;
-      e_chc = qc * m / rho;
-    }
-    double SR[6];
-    for (int k = 0; k < 6; ++k) SR[k] = d.sr[k * np + i];
-    const double ex = M.th_exp * dTdt;
-    for (int k = 0; k < 3; ++k) {
-      SR[k] += ex;
-      d.sr[k * np + i] = SR[k];
-    }
-    double S[6];
-    for (int k = 0; k < 6; ++k) S[k] = d.S[k * np + i];
-    e_int = voli * (S[XX] * SR[XX] + 2.0 * S[XY] * SR[XY] + 2.0 * S[XZ] * SR[XZ] + S[YY] * SR[YY] +
-                    2.0 * S[YZ] * SR[YZ] + S[ZZ] * SR[ZZ]);
+    e = thermal_own(d, buf, i, temp);
   }
-  const double r0 = block_reduce<0>(e_int, sh);
-  if (threadIdx.x == 0) part(d, P_INT, blockIdx.x) = r0;
-  if (d.qfric) {
-    const double r1 = block_reduce<0>(e_frw, sh);
-    const double r2 = block_reduce<0>(e_chc, sh);
-    if (threadIdx.x == 0) {
-      part(d, P_FRW, blockIdx.x) = r1;
-      part(d, P_CHC, blockIdx.x) = r2;
-    }
-  }
+  thermal_sums(d, e, t, sh);
 }
 
-void launch_thermal(const Dev &d, hipStream_t st, int buf, double dt) {
-  k_thermal<<<d.nblocks, kBlock, 0, st>>>(d, buf, dt);
+// records of the conduction gather: (x, y), (z, T), (m/rho, key)
+struct HeatLds {
+  const double2 *r;
+  __device__ void load(int p, double &x, double &y, double &z, double &T, double &vol, long long &key) const {
+    const double2 a = r[p], b = r[kStageMax + p], c = r[2 * kStageMax + p];
+    x = a.x, y = a.y, z = b.x, T = b.y, vol = c.x, key = __double_as_longlong(c.y);
+  }
+};
+struct HeatHbm {
+  const Dev &d;
+  const int buf;
+  __device__ void load(int j, double &x, double &y, double &z, double &T, double &vol, long long &key) const {
+    const double4 a = d.xh[buf][j];
+    x = a.x, y = a.y, z = a.z, T = d.T[j], vol = d.vol[buf][j], key = d.tkey[j];
+  }
+};
+constexpr int kLanesHeat = 2;
+template <class Rows, class Rec>
+__device__ inline double heat_lane(const Dev &d, int sub, int cnt, const double4 &xi, double Ti, double voli,
+                                   long long ki, const Rows &rows, typename Rows::G a0, typename Rows::G b0,
+                                   const Rec &rec) {
+  double s = 0.0;
+  const GkD k = gk_consts64(xi.w, d.dim);
+  walk_groups<kLanesHeat>(rows, cnt, sub, rows.self(), a0, b0, [&](const typename Rows::G &c) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      double x, y, z, T, vol;
+      long long key;
+      rec.load(entry(c, u), x, y, z, T, vol, key);
+      const double dx = xi.x - x, dy = xi.y - y, dz = xi.z - z;
+      const double GK = gk_d(dx * dx + dy * dy + dz * dz, k);
+      s = fma((key > ki ? vol : voli) * (Ti - T), GK, s);
+      if (u & 1) __builtin_amdgcn_sched_barrier(0);
+    }
+  });
+  return s;
+}
+__global__ __launch_bounds__(kBlock *kLanesHeat) void k_thermal_lds(Dev d, int buf) {
+  constexpr int NT = kBlock * kLanesHeat;
+  __shared__ double2 rec[3 * kStageMax];
+  __shared__ double red[(kLanesHeat - 1) * kBlock];
+  __shared__ double sh[NT / 64];
+  const int t = xcd_tile(blockIdx.x, gridDim.x), sub = threadIdx.x / kBlock;
+  const int i = t * kBlock + (int)(threadIdx.x % kBlock);
+  const int U = d.stage_cnt[t];
+  const bool on = i < d.n && d.group[i] >= 0;
+  const int cnt = on ? d.nnb[i] : 0;
+  const double4 xi = d.xh[buf][i];
+  const double Ti = d.T[i], voli = d.vol[buf][i];
+  const long long ki = d.tkey[i];
+  double s[1] = {0.0};
+  if (U < 0) {
+    const HbmRows rows{reinterpret_cast<const int4 *>(d.nbr) + i, d.npad, i};
+    if (on)
+      s[0] = heat_lane(d, sub, cnt, xi, Ti, voli, ki, rows, rows.group(2 * sub), rows.group(2 * sub + 1),
+                       HeatHbm{d, buf});
+  } else {
+    const LdsRows rows{reinterpret_cast<const ushort4 *>(d.nbrl) + i, d.npad, (int)d.selfl[i]};
+    const ushort4 a0 = rows.group(2 * sub), b0 = rows.group(2 * sub + 1);
+    const HeatHbm h{d, buf};
+    stage_set<NT>(d, t, U, [&](int p, int j) {
+      double x, y, z, T, vol;
+      long long key;
+      h.load(j, x, y, z, T, vol, key);
+      rec[p] = make_double2(x, y);
+      rec[kStageMax + p] = make_double2(z, T);
+      rec[2 * kStageMax + p] = make_double2(vol, __longlong_as_double(key));
+    });
+    if (on) s[0] = heat_lane(d, sub, cnt, xi, Ti, voli, ki, rows, a0, b0, HeatLds{rec});
+  }
+  combine_lanes<kLanesHeat>(s, red);
+  __builtin_amdgcn_sched_barrier(0);
+  double3 e = make_double3(0.0, 0.0, 0.0);
+  if (on && sub == 0) e = thermal_own(d, buf, i, pair_kk(d.mats[d.mat[i]]) * s[0]);
+  thermal_sums(d, e, t, sh);
+}
+
+void launch_thermal(const Dev &d, hipStream_t st, int buf) {
+  if (d.h_uni) k_thermal_lds<<<d.nblocks, kBlock * kLanesHeat, 0, st>>>(d, buf);
+  else k_thermal<<<d.nblocks, kBlock, 0, st>>>(d, buf);
 }
 
 // ---------------------------------------------------------------------------
