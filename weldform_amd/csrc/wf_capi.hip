@@ -1078,9 +1078,8 @@ void enqueue_step(Ctx *c, int scheme, int cur, const TapeHook *tp = nullptr, int
     }
     {
       Timed t(c, T_RATES);
-      launch_rates(d, c->st, nxt);
+      launch_rates(d, c->st, nxt, dt, 1);
     }
-    launch_stress(d, c->st, nxt, dt);
     if (c->cfg.thermal_solver) launch_thermal(d, c->st, nxt);
     launch_finalize(d, c->st, dt, c->bc.nz);
     if (d.contact) launch_mesh_update(d, c->st, dt);
@@ -2494,7 +2493,7 @@ int wf_eval(void *ctx, int32_t what, double dt) {
         launch_accel(c->d, c->st, c->cur);
         break;
       case WF_EVAL_DENSITY: launch_dens_drift(c->d, c->st, c->cur, dt, 0); break;
-      case WF_EVAL_RATES: launch_rates(c->d, c->st, c->cur); break;
+      case WF_EVAL_RATES: launch_rates(c->d, c->st, c->cur, 0.0, 0); break;
       case WF_EVAL_STRESS: launch_stress(c->d, c->st, c->cur, dt); break;
       default: throw Error(WF_EINVAL, "unknown evaluation");
     }

@@ -2313,8 +2313,8 @@ void launch_dens_drift(const Dev &d, hipStream_t st, int cur, double dt, int do_
 // stress update (Particle::CalcStressStrain, Source/Particle.cpp:960-1067)
 // with plastic work heat (Source/Particle.cpp:922-939), the temperature
 // update of ThermalCalcs (Source/Thermal.cpp:726-734) and the internal
-// energy term (Source/Domain.cpp:1810-1829).  The gather and the update are
-// separate kernels so the gather keeps a small register footprint.
+// energy term (Source/Domain.cpp:1810-1829).  The update is a kernel of its
+// own, or runs at the end of the gather kernel (see launch_rates).
 
 // one particle's rate-tensor gather: v[0..5] strain rate, v[6..8] rotation
 // rate (w01, w02, w12), v[9] the kinetic-energy pair sum
@@ -2367,19 +2367,241 @@ __device__ inline void rates_lane(const Dev &d, int buf, int i, const G &g, int 
 }
 
 template <typename R>
-__device__ inline double rates_store(const Dev &d, int i, const R (&v)[10]) {
+__device__ inline void rates_store(const Dev &d, int i, const R (&v)[10]) {
   const long long np = d.npad;
   for (int k = 0; k < 6; ++k) d.sr[k * np + i] = (double)v[k];
   for (int k = 0; k < 3; ++k) d.rr[k * np + i] = (double)v[6 + k];
-  return (double)v[9];
+}
+
+// Particle::CalcStressStrain and the per-particle terms after it for a free
+// particle with strain rate SR and rotation rate W
+struct StressSums {
+  double e_int = 0.0, e_plw = 0.0, tmax = -INFINITY, tmin = INFINITY;
+};
+// the state the update reads: the deviatoric stress (t), Sy, pl, T, rho and
+// m/rho, or in t the strain alone
+struct StressOwn {
+  double t[6], sigy, pl, T, rho, vol;
+};
+__device__ inline StressOwn stress_own(const Dev &d, int buf, int i) {
+  StressOwn o;
+  for (int k = 0; k < 6; ++k) o.t[k] = d.S[k * d.npad + i];
+  o.sigy = d.sigy[i];
+  o.pl = d.pl[i];
+  o.T = d.T[i];
+  o.rho = d.rho[buf][i];
+  o.vol = d.vol[buf][i];
+  return o;
+}
+__device__ inline void strain_update(const Dev &d, int i, double dt, const double (&SR)[6], const double (&strain)[6]) {
+  for (int k = 0; k < 6; ++k) d.strain[k * d.npad + i] = strain[k] + dt * SR[k];
+}
+template <bool MX>
+__device__ inline void stress_update(const Dev &d, int i, double dt, const double (&SR)[6], const double (&W)[3],
+                                     const StressOwn &o, StressSums &e) {
+  const long long np = d.npad;
+  const DevMat &M = d.mats[d.mat[i]];
+  const double rho = o.rho;
+  const double P = M.P0 + (M.Cs * M.Cs) * (rho - M.ref_density);
+  const double (&S)[6] = o.t;
+  // Jaumann terms S*W^T + W*S with W antisymmetric
+  const double Sf[3][3] = {{S[XX], S[XY], S[XZ]}, {S[XY], S[YY], S[YZ]}, {S[XZ], S[YZ], S[ZZ]}};
+  const double Wf[3][3] = {{0.0, W[0], W[1]}, {-W[0], 0.0, W[2]}, {-W[1], -W[2], 0.0}};
+  const int ia[6] = {0, 1, 2, 0, 0, 1}, ib[6] = {0, 1, 2, 1, 2, 2};
+  const double c3 = 1.0 / 3.0 * (SR[XX] + SR[YY] + SR[ZZ]);
+  const double G2 = 2.0 * M.G;
+  double Sn[6];
+  for (int k = 0; k < 6; ++k) {
+    const int a = ia[k], b = ib[k];
+    double jt = 0.0;
+    for (int q = 0; q < 3; ++q) jt += Sf[a][q] * Wf[b][q] + Wf[a][q] * Sf[q][b];
+    const double dev = k < 3 ? SR[k] - c3 : SR[k];
+    Sn[k] = dt * (G2 * dev + jt) + S[k];
+  }
+  const double effsr = sqrt(0.5 * ((SR[XX] - SR[YY]) * (SR[XX] - SR[YY]) + (SR[YY] - SR[ZZ]) * (SR[YY] - SR[ZZ]) +
+                                   (SR[ZZ] - SR[XX]) * (SR[ZZ] - SR[XX])) +
+                            3.0 * (SR[XY] * SR[XY] + SR[YZ] * SR[YZ] + SR[XZ] * SR[XZ]));
+  const double J2 = 0.5 * (Sn[XX] * Sn[XX] + 2.0 * Sn[XY] * Sn[XY] + 2.0 * Sn[XZ] * Sn[XZ] + Sn[YY] * Sn[YY] +
+                           2.0 * Sn[YZ] * Sn[YZ] + Sn[ZZ] * Sn[ZZ]);
+  const double sig_trial = sqrt(3.0 * J2);
+  double Sy = o.sigy;
+  double pl = o.pl;
+  const double ratio = Sy / sig_trial;
+  const double fac = (1.0 < ratio) ? 1.0 : ratio;
+  for (int k = 0; k < 6; ++k) Sn[k] *= fac;
+  const double T = o.T;
+  if (M.model == WF_HOLLOMON) Sy = hol_yield(M, pl);
+  else if (M.model == WF_JOHNSON_COOK) Sy = jc_yield(M, pl, effsr, T);
+  double dep = 0.0;
+  if (sig_trial > Sy) {
+    dep = (sig_trial - Sy) / (3. * M.G + M.Ep);
+    pl += dep;
+    d.dpl[i] = dep;
+    if (M.model == WF_BILINEAR) Sy += dep * M.Ep;
+  }
+  double sig[6];
+  for (int k = 0; k < 6; ++k) sig[k] = k < 3 ? -P + Sn[k] : Sn[k];
+  if (dep > 0.0) {
+    const double f = dep / Sy;
+    const double inc[6] = {f * (sig[XX] - 0.5 * (sig[YY] + sig[ZZ])), f * (sig[YY] - 0.5 * (sig[XX] + sig[ZZ])),
+                           f * (sig[ZZ] - 0.5 * (sig[XX] + sig[YY])), 1.5 * f * sig[XY],
+                           1.5 * f * sig[XZ],                          1.5 * f * sig[YZ]};
+    for (int k = 0; k < 6; ++k) {
+      d.eplinc[k * np + i] = inc[k];
+      d.epl[k * np + i] += inc[k];
+    }
+  }
+  for (int k = 0; k < 6; ++k) d.S[k * np + i] = Sn[k];
+  d.effsr[i] = effsr;
+  d.sigy[i] = Sy;
+  d.pl[i] = pl;
+  d.pres[i] = P;
+  // Domain::CalcDamage, Johnson-Cook criterion (Source/Damage.cpp:9-46),
+  // after the stress update: the (never reset) delta_pl_strain over the
+  // fracture strain at the plastic rate, the triaxiality -P / Sigma_eq
+  // (Particle::CalculateEquivalentStress, Source/Particle.cpp:623-633)
+  // and T (0 without the thermal solver: the reference's is an
+  // uninitialised private copy of a local set to 0)
+  if (d.damage && M.dam_model == 1) {
+    const double dpl = d.dpl[i];
+    if (dpl > 0.0) {
+      const double J2e = 0.5 * (Sn[XX] * Sn[XX] + 2.0 * Sn[XY] * Sn[XY] + 2.0 * Sn[XZ] * Sn[XZ] + Sn[YY] * Sn[YY] +
+                                2.0 * Sn[YZ] * Sn[YZ] + Sn[ZZ] * Sn[ZZ]);
+      const double seq = sqrt(3.0 * J2e);
+      if (seq > 1.0e-3) {
+        const double ef = jc_fracture_strain(M, dpl / dt, -P / seq, d.thermal ? T : 0.0);
+        double D = d.damD[i] + dpl / ef;
+        if (D > 1.0) D = 1.0;
+        d.damD[i] = D;
+      }
+    }
+  }
+  if (pl > 1.e-6) d.flags->yielded = 1;
+  StressRec rec;
+  for (int k = 0; k < 6; ++k) rec.s[k] = sig[k];
+  rec.rho = rho;
+  rec.irho2 = 1.0 / (rho * rho);
+  d.srec[i] = rec;
+  if (MX) {
+    StressRecF rf;
+    for (int k = 0; k < 6; ++k) rf.t[k] = (float)(sig[k] * rec.irho2);
+    rf.rho = (float)rho;
+    rf.pad = 0.0f;
+    d.srecf[i] = rf;
+  }
+  const double vol = o.vol;
+  // plastic work heat, Source/ThermalStuct.cpp:14-39 (delta_pl_strain is
+  // never reset by the reference, so the last increment keeps heating)
+  if (d.pl_heating) {
+    double q = d.qpl[i];
+    if (d.dpl[i] > 0.0) {
+      double dp[6];
+      for (int k = 0; k < 6; ++k) dp[k] = d.eplinc[k * np + i] * (1. / dt);
+      q = sig[XX] * dp[XX] + 2.0 * sig[XY] * dp[XY] + 2.0 * sig[XZ] * dp[XZ] + sig[YY] * dp[YY] +
+          2.0 * sig[YZ] * dp[YZ] + sig[ZZ] * dp[ZZ];
+      d.qpl[i] = q;
+    }
+    d.psen[i] += q * dt;
+    e.e_plw = vol * q;
+  }
+  if (d.thermal) {
+    const double Tn = T + dt * d.dTdt[i];
+    d.T[i] = Tn;
+    e.tmax = Tn;
+    e.tmin = Tn;
+  } else {
+    e.e_int = vol * (Sn[XX] * SR[XX] + 2.0 * Sn[XY] * SR[XY] + 2.0 * Sn[XZ] * SR[XZ] + Sn[YY] * SR[YY] +
+                   2.0 * Sn[YZ] * SR[YZ] + Sn[ZZ] * SR[ZZ]);
+  }
+}
+
+// block partials of the energies, plastic work and temperature range; the
+// particles are the block's first kBlock threads (every thread calls this;
+// sh: 5 * kBlock / 64 values)
+template <bool KIN, bool STRESS>
+__device__ inline void rates_sums(const Dev &d, int t, double e_kin, const StressSums &e, double *sh) {
+  constexpr int NW = kBlock / 64;
+  const int w = threadIdx.x >> 6;
+  if (w < NW) {
+    const double r[5] = {KIN ? wave_sum(e_kin) : 0.0, STRESS ? wave_sum(e.e_int) : 0.0,
+                         STRESS ? wave_sum(e.e_plw) : 0.0, STRESS ? wave_max(e.tmax) : 0.0,
+                         STRESS ? wave_min(e.tmin) : 0.0};
+    if ((threadIdx.x & 63) == 0)
+      for (int q = 0; q < 5; ++q) sh[q * NW + w] = r[q];
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  static_assert(NW == 2, "two wavefronts of particles per block");
+  if (KIN) part(d, P_KIN, t) = sh[0] + sh[1];
+  if (STRESS) {
+    part(d, P_INT, t) = sh[2] + sh[3];
+    part(d, P_PLW, t) = sh[4] + sh[5];
+    part(d, P_MAXT, t) = fmax(sh[6], sh[7]);
+    part(d, P_MINT, t) = fmin(sh[8], sh[9]);
+  }
+}
+
+// The rate passes' end.  Every lane's partial sums meet in LDS (red: LANES *
+// 10 * kBlock values, the staged records' space) and are added in lane order;
+// lane 0 of the particle then runs the stress update, lane 1 (with one lane,
+// the same) stores the rates and updates the strain.  Both parts' inputs are
+// loaded by rates_pre before the tile is staged, so that they arrive during
+// the row walk.
+template <int LANES>
+__device__ inline StressOwn rates_pre(const Dev &d, int buf, int i, int sub, int do_stress) {
+  StressOwn o{};
+  if (!do_stress || i >= d.n) return o;
+  if (sub == 0) o = stress_own(d, buf, i);
+  else if (sub == 1)
+    for (int k = 0; k < 6; ++k) o.t[k] = d.strain[k * d.npad + i];
+  return o;
+}
+template <bool MX, int LANES, typename R>
+__device__ inline void rates_finish(const Dev &d, int i, int sub, R (&v)[10], const StressOwn &o, double dt,
+                                    int do_stress, R *red, double *sh) {
+  const int lane = threadIdx.x % kBlock;
+  if constexpr (LANES > 1) {
+    __syncthreads();  // the staged records are read before the sums overwrite them
+    for (int c = 0; c < 10; ++c) red[(sub * 10 + c) * kBlock + lane] = v[c];
+    __syncthreads();
+    if (sub < 2)
+      for (int c = 0; c < 10; ++c) {
+        R r = red[c * kBlock + lane];
+        for (int q = 1; q < LANES; ++q) r += red[(q * 10 + c) * kBlock + lane];
+        v[c] = r;
+      }
+  }
+  double e_kin = 0.0;
+  StressSums e;
+  if (sub < 2 && i < d.n) {
+    const bool stress = do_stress && d.group[i] >= 0;
+    if (dt < 0) dt = d.flags->dt;
+    const double SR[6] = {(double)v[0], (double)v[1], (double)v[2], (double)v[3], (double)v[4], (double)v[5]};
+    const double W[3] = {(double)v[6], (double)v[7], (double)v[8]};
+    if (sub == LANES - 1 || sub == 1) {
+      rates_store(d, i, v);
+      if (stress) {
+        double strain[6];
+        for (int k = 0; k < 6; ++k) strain[k] = LANES == 1 ? d.strain[k * d.npad + i] : o.t[k];
+        strain_update(d, i, dt, SR, strain);
+      }
+    }
+    if (sub == 0) {
+      e_kin = (double)v[9];
+      if (stress) stress_update<MX>(d, i, dt, SR, W, o, e);
+    }
+  }
+  if (do_stress) rates_sums<true, true>(d, blockIdx.x, e_kin, e, sh);
+  else rates_sums<true, false>(d, blockIdx.x, e_kin, e, sh);
 }
 
 template <int LANES>
-__global__ __launch_bounds__(kBlock *LANES) void k_rates_f64(Dev d, int buf) {
-  __shared__ double red[(LANES > 1 ? LANES - 1 : 1) * 10 * kBlock];
-  __shared__ double sh[kBlock * LANES / 64];
+__global__ __launch_bounds__(kBlock *LANES) void k_rates_f64(Dev d, int buf, double dt, int do_stress) {
+  __shared__ double red[LANES > 1 ? LANES * 10 * kBlock : 1];
+  __shared__ double sh[5 * kBlock / 64];
   const int t = xcd_tile(blockIdx.x, gridDim.x), sub = threadIdx.x / kBlock;
   const int i = t * kBlock + (int)(threadIdx.x % kBlock);
+  const StressOwn own = rates_pre<LANES>(d, buf, i, sub, do_stress);
   double v[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   if (i < d.n) {
     const HbmJ<false> g{d, buf, i};
@@ -2391,26 +2613,24 @@ __global__ __launch_bounds__(kBlock *LANES) void k_rates_f64(Dev d, int buf) {
       else rates_lane<false, false>(d, buf, i, g, sub, LANES, v);
     }
   }
-  combine_lanes<LANES>(v, red);
-  const double e_kin = (i < d.n && sub == 0) ? rates_store(d, i, v) : 0.0;
-  const double r1 = block_reduce<0>(e_kin, sh);
-  if (threadIdx.x == 0) part(d, P_KIN, blockIdx.x) = r1;
+  rates_finish<false, LANES>(d, i, sub, v, own, dt, do_stress, red, sh);
 }
 
 // FP64, uniform h: 72 bytes of LDS per staged particle, two blocks per CU;
 // the lanes' partial sums reuse the records' space
 template <bool GC>
-__global__ __launch_bounds__(kBlock *kLanesLds64) void k_rates64(Dev d, int buf) {
+__global__ __launch_bounds__(kBlock *kLanesLds64) __attribute__((amdgpu_waves_per_eu(4))) void k_rates64(Dev d, int buf, double dt, int do_stress) {
   __shared__ double2 rec[kRecRates * kStageMax];
   __shared__ double sc[kStageMax];
-  static_assert(2 * kRecRates * kStageMax >= (kLanesLds64 - 1) * 10 * kBlock, "the partial sums fit the records' space");
-  __shared__ double sh[kBlock * kLanesLds64 / 64];
+  static_assert(2 * kRecRates * kStageMax >= kLanesLds64 * 10 * kBlock, "the partial sums fit the records' space");
+  __shared__ double sh[5 * kBlock / 64];
   const int t = xcd_tile(blockIdx.x, gridDim.x), sub = threadIdx.x / kBlock;
   const int i = t * kBlock + (int)(threadIdx.x % kBlock);
   const int U = d.stage_cnt[t];
   const bool on = i < d.n && d.group[i] >= 0;
   const int cnt = on ? d.nnb[i] : 0;
   const double4 xi = d.xh[buf][i], vi = d.vm[i];
+  const StressOwn own = rates_pre<kLanesLds64>(d, buf, i, sub, do_stress);
   double v[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   if (U < 0) {
     const HbmRows rows{reinterpret_cast<const int4 *>(d.nbr) + i, d.npad, i};
@@ -2424,11 +2644,7 @@ __global__ __launch_bounds__(kBlock *kLanesLds64) void k_rates64(Dev d, int buf)
     const RecLds64<PASS_RATES> l{rec, sc, nullptr};
     if (on) rates64_lane<GC>(d, i, rows.own, sub, cnt, xi, vi, l.pr(rows.own), rows, a0, b0, l, v);
   }
-  __syncthreads();  // the records are read before the partial sums overwrite them
-  combine_lanes<kLanesLds64>(v, reinterpret_cast<double *>(rec));
-  const double e_kin = (i < d.n && sub == 0) ? rates_store(d, i, v) : 0.0;
-  const double r1 = block_reduce<0>(e_kin, sh);
-  if (threadIdx.x == 0) part(d, P_KIN, blockIdx.x) = r1;
+  rates_finish<false, kLanesLds64>(d, i, sub, v, own, dt, do_stress, reinterpret_cast<double *>(rec), sh);
 }
 
 // CalcRateTensors + RateTensorsReduction in FP32
@@ -2497,14 +2713,16 @@ __device__ inline void rates_mx_lane(const Dev &d, int buf, int i, int own, int 
 }
 
 template <int LANES, bool GC>
-__global__ __launch_bounds__(kBlock *LANES) void k_rates_mx(Dev d, int buf) {
-  __shared__ float4 lx[kStageMax + 1], lv[kStageMax + 1];
+__global__ __launch_bounds__(kBlock *LANES) void k_rates_mx(Dev d, int buf, double dt, int do_stress) {
+  __shared__ float4 lx[2 * (kStageMax + 1)];
   __shared__ float lp[kStageMax + 1];
-  __shared__ float red[(LANES > 1 ? LANES - 1 : 1) * 10 * kBlock];
-  __shared__ double sh[kBlock * LANES / 64];
+  float4 *lv = lx + kStageMax + 1;
+  static_assert(8 * (kStageMax + 1) >= LANES * 10 * kBlock, "the partial sums fit the records' space");
+  __shared__ double sh[5 * kBlock / 64];
   const int t = xcd_tile(blockIdx.x, gridDim.x), sub = threadIdx.x / kBlock;
   const int i = t * kBlock + (int)(threadIdx.x % kBlock);
   const int U = d.stage_cnt[t];
+  const StressOwn own = rates_pre<LANES>(d, buf, i, sub, do_stress);
   float v[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   if (U < 0) {
     if (i < d.n && d.group[i] >= 0) {
@@ -2518,166 +2736,50 @@ __global__ __launch_bounds__(kBlock *LANES) void k_rates_mx(Dev d, int buf) {
       rates_mx_lane<LANES, GC, true>(d, buf, i, d.selfl[i], sub, rows, XvLds{lx, lv, lp}, v);
     }
   }
-  combine_lanes<LANES>(v, red);
-  const double e_kin = (i < d.n && sub == 0) ? rates_store(d, i, v) : 0.0;
-  const double r1 = block_reduce<0>(e_kin, sh);
-  if (threadIdx.x == 0) part(d, P_KIN, blockIdx.x) = r1;
+  rates_finish<true, LANES>(d, i, sub, v, own, dt, do_stress, reinterpret_cast<float *>(lx), sh);
 }
 
+// the stress update alone (single-pass evaluations)
 template <bool MX>
 WF_KERNEL void k_stress(Dev d, int buf, double dt) {
-  if (dt < 0) dt = d.flags->dt;
-  __shared__ double sh[kBlock / 64];
+  __shared__ double sh[5 * kBlock / 64];
   const int i = blockIdx.x * kBlock + threadIdx.x;
   const long long np = d.npad;
-  double e_int = 0.0, e_plw = 0.0, tmax = -INFINITY, tmin = INFINITY;
-  if (i < d.n) {
-    const int g = d.group[i];
+  StressSums e;
+  if (i < d.n && d.group[i] >= 0) {
     double SR[6], W[3];
     for (int k = 0; k < 6; ++k) SR[k] = d.sr[k * np + i];
     for (int k = 0; k < 3; ++k) W[k] = d.rr[k * np + i];
-    if (g >= 0) {
-      const DevMat &M = d.mats[d.mat[i]];
-      const double rho = d.rho[buf][i];
-      const double P = M.P0 + (M.Cs * M.Cs) * (rho - M.ref_density);
-      double S[6];
-      for (int k = 0; k < 6; ++k) S[k] = d.S[k * np + i];
-      // Jaumann terms S*W^T + W*S with W antisymmetric
-      const double Sf[3][3] = {{S[XX], S[XY], S[XZ]}, {S[XY], S[YY], S[YZ]}, {S[XZ], S[YZ], S[ZZ]}};
-      const double Wf[3][3] = {{0.0, W[0], W[1]}, {-W[0], 0.0, W[2]}, {-W[1], -W[2], 0.0}};
-      const int ia[6] = {0, 1, 2, 0, 0, 1}, ib[6] = {0, 1, 2, 1, 2, 2};
-      const double c3 = 1.0 / 3.0 * (SR[XX] + SR[YY] + SR[ZZ]);
-      const double G2 = 2.0 * M.G;
-      double Sn[6];
-      for (int k = 0; k < 6; ++k) {
-        const int a = ia[k], b = ib[k];
-        double jt = 0.0;
-        for (int q = 0; q < 3; ++q) jt += Sf[a][q] * Wf[b][q] + Wf[a][q] * Sf[q][b];
-        const double dev = k < 3 ? SR[k] - c3 : SR[k];
-        Sn[k] = dt * (G2 * dev + jt) + S[k];
-      }
-      const double effsr = sqrt(0.5 * ((SR[XX] - SR[YY]) * (SR[XX] - SR[YY]) + (SR[YY] - SR[ZZ]) * (SR[YY] - SR[ZZ]) +
-                                       (SR[ZZ] - SR[XX]) * (SR[ZZ] - SR[XX])) +
-                                3.0 * (SR[XY] * SR[XY] + SR[YZ] * SR[YZ] + SR[XZ] * SR[XZ]));
-      const double J2 = 0.5 * (Sn[XX] * Sn[XX] + 2.0 * Sn[XY] * Sn[XY] + 2.0 * Sn[XZ] * Sn[XZ] + Sn[YY] * Sn[YY] +
-                               2.0 * Sn[YZ] * Sn[YZ] + Sn[ZZ] * Sn[ZZ]);
-      const double sig_trial = sqrt(3.0 * J2);
-      double Sy = d.sigy[i];
-      double pl = d.pl[i];
-      const double ratio = Sy / sig_trial;
-      const double fac = (1.0 < ratio) ? 1.0 : ratio;
-      for (int k = 0; k < 6; ++k) Sn[k] *= fac;
-      const double T = d.T[i];
-      if (M.model == WF_HOLLOMON) Sy = hol_yield(M, pl);
-      else if (M.model == WF_JOHNSON_COOK) Sy = jc_yield(M, pl, effsr, T);
-      double dep = 0.0;
-      if (sig_trial > Sy) {
-        dep = (sig_trial - Sy) / (3. * M.G + M.Ep);
-        pl += dep;
-        d.dpl[i] = dep;
-        if (M.model == WF_BILINEAR) Sy += dep * M.Ep;
-      }
-      double sig[6];
-      for (int k = 0; k < 6; ++k) sig[k] = k < 3 ? -P + Sn[k] : Sn[k];
-      if (dep > 0.0) {
-        const double f = dep / Sy;
-        const double inc[6] = {f * (sig[XX] - 0.5 * (sig[YY] + sig[ZZ])), f * (sig[YY] - 0.5 * (sig[XX] + sig[ZZ])),
-                               f * (sig[ZZ] - 0.5 * (sig[XX] + sig[YY])), 1.5 * f * sig[XY],
-                               1.5 * f * sig[XZ],                          1.5 * f * sig[YZ]};
-        for (int k = 0; k < 6; ++k) {
-          d.eplinc[k * np + i] = inc[k];
-          d.epl[k * np + i] += inc[k];
-        }
-      }
-      for (int k = 0; k < 6; ++k) {
-        d.S[k * np + i] = Sn[k];
-        d.strain[k * np + i] += dt * SR[k];
-      }
-      d.effsr[i] = effsr;
-      d.sigy[i] = Sy;
-      d.pl[i] = pl;
-      d.pres[i] = P;
-      // Domain::CalcDamage, Johnson-Cook criterion (Source/Damage.cpp:9-46),
-      // after the stress update: the (never reset) delta_pl_strain over the
-      // fracture strain at the plastic rate, the triaxiality -P / Sigma_eq
-      // (Particle::CalculateEquivalentStress, Source/Particle.cpp:623-633)
-      // and T (0 without the thermal solver: the reference's is an
-      // uninitialised private copy of a local set to 0)
-      if (d.damage && M.dam_model == 1) {
-        const double dpl = d.dpl[i];
-        if (dpl > 0.0) {
-          const double J2e = 0.5 * (Sn[XX] * Sn[XX] + 2.0 * Sn[XY] * Sn[XY] + 2.0 * Sn[XZ] * Sn[XZ] + Sn[YY] * Sn[YY] +
-                                    2.0 * Sn[YZ] * Sn[YZ] + Sn[ZZ] * Sn[ZZ]);
-          const double seq = sqrt(3.0 * J2e);
-          if (seq > 1.0e-3) {
-            const double ef = jc_fracture_strain(M, dpl / dt, -P / seq, d.thermal ? T : 0.0);
-            double D = d.damD[i] + dpl / ef;
-            if (D > 1.0) D = 1.0;
-            d.damD[i] = D;
-          }
-        }
-      }
-      if (pl > 1.e-6) d.flags->yielded = 1;
-      StressRec rec;
-      for (int k = 0; k < 6; ++k) rec.s[k] = sig[k];
-      rec.rho = rho;
-      rec.irho2 = 1.0 / (rho * rho);
-      d.srec[i] = rec;
-      if (MX) {
-        StressRecF rf;
-        for (int k = 0; k < 6; ++k) rf.t[k] = (float)(sig[k] * rec.irho2);
-        rf.rho = (float)rho;
-        rf.pad = 0.0f;
-        d.srecf[i] = rf;
-      }
-      const double vol = d.vol[buf][i];
-      // plastic work heat, Source/ThermalStuct.cpp:14-39 (delta_pl_strain is
-      // never reset by the reference, so the last increment keeps heating)
-      if (d.pl_heating) {
-        double q = d.qpl[i];
-        if (d.dpl[i] > 0.0) {
-          double dp[6];
-          for (int k = 0; k < 6; ++k) dp[k] = d.eplinc[k * np + i] * (1. / dt);
-          q = sig[XX] * dp[XX] + 2.0 * sig[XY] * dp[XY] + 2.0 * sig[XZ] * dp[XZ] + sig[YY] * dp[YY] +
-              2.0 * sig[YZ] * dp[YZ] + sig[ZZ] * dp[ZZ];
-          d.qpl[i] = q;
-        }
-        d.psen[i] += q * dt;
-        e_plw = vol * q;
-      }
-      if (d.thermal) {
-        const double Tn = T + dt * d.dTdt[i];
-        d.T[i] = Tn;
-        tmax = Tn;
-        tmin = Tn;
-      } else {
-        e_int = vol * (Sn[XX] * SR[XX] + 2.0 * Sn[XY] * SR[XY] + 2.0 * Sn[XZ] * SR[XZ] + Sn[YY] * SR[YY] +
-                       2.0 * Sn[YZ] * SR[YZ] + Sn[ZZ] * SR[ZZ]);
-      }
-    }
+    double strain[6];
+    for (int k = 0; k < 6; ++k) strain[k] = d.strain[k * np + i];
+    strain_update(d, i, dt, SR, strain);
+    stress_update<MX>(d, i, dt, SR, W, stress_own(d, buf, i), e);
   }
-  const double r0 = block_reduce<0>(e_int, sh);
-  const double r2 = block_reduce<0>(e_plw, sh);
-  const double r3 = block_reduce<1>(tmax, sh);
-  const double r4 = block_reduce<2>(tmin, sh);
-  if (threadIdx.x == 0) {
-    part(d, P_INT, blockIdx.x) = r0;
-    part(d, P_PLW, blockIdx.x) = r2;
-    part(d, P_MAXT, blockIdx.x) = r3;
-    part(d, P_MINT, blockIdx.x) = r4;
-  }
+  rates_sums<false, true>(d, blockIdx.x, 0.0, e, sh);
 }
 
-void launch_rates(const Dev &d, hipStream_t st, int buf) {
+// The stress update runs inside the rate kernel up to about one tile per CU:
+// there a launch costs more than what the update's dependent chain (return
+// map, powers) adds to each block.  Above, a kernel of its own keeps more of
+// those chains in flight.  Rates and update, fused against apart: 1.3k
+// particles 11.3 and 15.5 us, 35k 16.2 and 22.7; 56k (FP64) 26.6 and 32, but a
+// damage step 2 % slower; 370k 84 and 85, 954k 200 and 194 (FP64 301 and 272).
+constexpr int kFuseTiles = 320;
+void launch_rates(const Dev &d, hipStream_t st, int buf, double dt, int do_stress) {
+  if (do_stress && d.ntiles > kFuseTiles) {
+    launch_rates(d, st, buf, dt, 0);
+    launch_stress(d, st, buf, dt);
+    return;
+  }
   if (d.mixed) {
-    WF_LANES_GC_SWITCH(d.lanes_mx, d.gc_on, k_rates_mx, d, buf)
+    WF_LANES_GC_SWITCH(d.lanes_mx, d.gc_on, k_rates_mx, d, buf, dt, do_stress)
   } else {
     if (d.lds64) {
       gc_switch(d.gc_on, [&](auto gc) {
-        k_rates64<decltype(gc)::value><<<nblk(d.n), kBlock * kLanesLds64, 0, st>>>(d, buf);
+        k_rates64<decltype(gc)::value><<<nblk(d.n), kBlock * kLanesLds64, 0, st>>>(d, buf, dt, do_stress);
       });
     } else {
-      WF_LANES_SWITCH(d.lanes_f64, k_rates_f64, d, buf)
+      WF_LANES_SWITCH(d.lanes_f64, k_rates_f64, d, buf, dt, do_stress)
     }
   }
 }
