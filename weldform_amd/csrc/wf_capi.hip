@@ -999,7 +999,8 @@ void enqueue_step(Ctx *c, int scheme, int cur, const TapeHook *tp = nullptr, int
     // (Source/SolverLeapfrog.cpp:126, Source/SolverKickDrift.cpp:119)
     if (d.dim == 2) launch_plane_strain(d, c->st);
     if (tp) tape_state(c, tp->s, cur);
-    launch_schedule(d, c->st, 0);
+    // (in a step run in parts the rigid planes take theirs with the contact)
+    launch_schedule(d, c->st, 0, split ? nullptr : &c->bc);
     {
       Timed t(c, T_NBR);
       launch_neighbours(d, c->st, cur);
@@ -1031,7 +1032,8 @@ void enqueue_step(Ctx *c, int scheme, int cur, const TapeHook *tp = nullptr, int
     // so no BC zone applies to them
     // SolveDiffUpdateKickDrift calls Wang's law whatever contact_alg says
     // (Source/SolverKickDrift.cpp:211)
-    if (d.contact) launch_contact(d, c->st, c->bc, cur, dt, scheme == WF_LEAPFROG ? d.contact_law : 1);
+    if (d.contact && split) launch_rigid_bc(d, c->st, c->bc);
+    if (d.contact) launch_contact(d, c->st, cur, dt, scheme == WF_LEAPFROG ? d.contact_law : 1);
     if (d.contact && d.ngroups > 0) launch_group_sums(d, c->st, 1);
     if (tp && d.contact) {
       d2d(c, tp->s.node, d.node, (size_t)d.nnode * sizeof(double4));
@@ -1065,7 +1067,7 @@ void enqueue_step(Ctx *c, int scheme, int cur, const TapeHook *tp = nullptr, int
         launch_dens_drift(d, c->st, cur, dt, 1);
       }
       launch_kick2(d, c->st, dt);
-      if (d.contact) launch_rigid_drift(d, c->st, dt);
+      if (d.contact && split) launch_rigid_drift(d, c->st, dt);
     }
   }
   if (in(P_REST)) {
@@ -1074,15 +1076,14 @@ void enqueue_step(Ctx *c, int scheme, int cur, const TapeHook *tp = nullptr, int
         Timed t(c, T_DENS);
         launch_dens_drift(d, c->st, cur, dt, 1);
       }
-      if (d.contact) launch_rigid_drift(d, c->st, dt);
+      if (d.contact && split) launch_rigid_drift(d, c->st, dt);
     }
     {
       Timed t(c, T_RATES);
       launch_rates(d, c->st, nxt, dt, 1);
     }
     if (c->cfg.thermal_solver) launch_thermal(d, c->st, nxt);
-    launch_finalize(d, c->st, dt, c->bc.nz);
-    if (d.contact) launch_mesh_update(d, c->st, dt);
+    launch_finalize(d, c->st, dt, c->bc.nz, split ? 0 : 1);
     if (tp) {
       d2d(c, tp->s.sr, d.sr, 6 * np * sizeof(double));
       d2d(c, tp->s.rr, d.rr, 3 * np * sizeof(double));
@@ -1807,7 +1808,7 @@ int wf_init(void *ctx, double dt) {
     if (c->d.contact) {
       // free surface before the loop (Source/SolverLeapfrog.cpp:84-100)
       refresh_bc(c);
-      launch_schedule(c->d, c->st, 1);
+      launch_schedule(c->d, c->st, 1, nullptr);
       launch_neighbours(c->d, c->st, 0);
       launch_surface(c->d, c->st, 0, 1);
     }
@@ -2444,7 +2445,7 @@ int wf_rebuild_neighbours(void *ctx) {
   return guard(c, [&] {
     as_ctx(ctx);
     if (!c->inited) throw Error(WF_ESTATE, "wf_init not called");
-    launch_schedule(c->d, c->st, 1);
+    launch_schedule(c->d, c->st, 1, nullptr);
     launch_neighbours(c->d, c->st, c->cur);
     if (c->d.gc_on) launch_gradcorr(c->d, c->st, c->cur);
     HIPCHK(hipGetLastError());

@@ -363,7 +363,8 @@ void launch_adj_reduce(const Dev &d, hipStream_t st, const AdjBufs &b, double *o
 void launch_tape_lists(const Dev &d, hipStream_t st, const AdjSlot &s, int force, int *ver, int slot);
 
 // launchers (wf_kernels.hip); all enqueue on `st`
-void launch_schedule(const Dev &d, hipStream_t st, int force);
+// bc: with the velocities of the rigid planes at the step's time
+void launch_schedule(const Dev &d, hipStream_t st, int force, const BcTable *bc);
 void launch_plane_strain(const Dev &d, hipStream_t st);
 void launch_neighbours(const Dev &d, hipStream_t st, int cur);
 void launch_gradcorr(const Dev &d, hipStream_t st, int cur);
@@ -386,19 +387,21 @@ void launch_dens_drift(const Dev &d, hipStream_t st, int cur, double dt, int do_
 void launch_rates(const Dev &d, hipStream_t st, int buf, double dt, int do_stress);
 void launch_stress(const Dev &d, hipStream_t st, int buf, double dt);
 void launch_thermal(const Dev &d, hipStream_t st, int buf);
-void launch_finalize(const Dev &d, hipStream_t st, double dt, int nz);
+// the end-of-step sums and the rigid meshes' update; drift: with the rigid
+// particles' drift before it
+void launch_finalize(const Dev &d, hipStream_t st, double dt, int nz, int drift);
 void launch_max_pl(const Dev &d, hipStream_t st);
 void launch_shadows(const Dev &d, hipStream_t st, int cur);
 void launch_surface(const Dev &d, hipStream_t st, int cur, int setup);
 // Domain::CalcForce2233 over every particle's row (FP64)
 void launch_force2233(const Dev &d, hipStream_t st, int cur, double xsph, int shepard);
 // law: Domain::contact_alg (0 Fraser, 1 Wang, 2 Seo, 4 LSDyna)
-void launch_contact(const Dev &d, hipStream_t st, const BcTable &bc, int cur, double dt, int law);
+void launch_rigid_bc(const Dev &d, hipStream_t st, const BcTable &bc);
+void launch_contact(const Dev &d, hipStream_t st, int cur, double dt, int law);
 // per-group sums of the step: what 0 the zone reaction (after the
 // acceleration pass), 1 the contact forces per mesh (after contact)
 void launch_group_sums(const Dev &d, hipStream_t st, int what);
 void launch_rigid_drift(const Dev &d, hipStream_t st, double dt);
-void launch_mesh_update(const Dev &d, hipStream_t st, double dt);
 // output tables (wf_output.hip)
 void launch_pack_xdmf(const Dev &d, hipStream_t st, int cur, float *f, int *iv);
 void launch_pack_csv(const Dev &d, hipStream_t st, int cur, double *rows);

@@ -77,10 +77,42 @@ __device__ inline int cell_coord(double x, double blpf, double cs, int cn) {
   return (int)f;
 }
 
+// velocity of each plane and of its particles at the step's time
+// (UserAcc's BC loop and the contact-mesh branch, Source/WeldForm.cpp:67-119)
+__device__ inline void rigid_bc(const Dev &d, const BcTable &bc, int r) {
+  if (r >= d.nrig) return;
+  const int m = d.rmesh[r];
+  const int zone = d.mesh_zone[m];
+  bool set = false, wset = false;
+  double v[3] = {0, 0, 0}, w[3] = {0, 0, 0};
+  for (int b = 0; b < bc.n; ++b) {
+    if (bc.zone[b] != zone || bc.type[b] != 0) continue;
+    if (bc.value_type[b] == 1) {
+      if (bc.amp[b] < 0) continue;
+      const double f = bc.amp_factor[b] * amp_value(d.amps[bc.amp[b]], d.flags->time);
+      for (int k = 0; k < 3; ++k) v[k] = f * bc.v[b][k];
+    } else {
+      for (int k = 0; k < 3; ++k) v[k] = bc.v[b][k];
+      // SetRotAxisVel: constant BCs only (Source/WeldForm.cpp:97-101)
+      for (int k = 0; k < 3; ++k) w[k] = bc.w[b][k];
+      wset = true;
+    }
+    set = true;
+  }
+  if (!set) return;
+  d.rv[r] = make_double4(v[0], v[1], v[2], 0.0);
+  if (r == d.mesh_elem0[m]) {
+    d.mv[m] = make_double4(v[0], v[1], v[2], 0.0);
+    if (wset) d.mw[m] = make_double4(w[0], w[1], w[2], 0.0);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // neighbour schedule (Source/SolverLeapfrog.cpp:160-201, 347-356)
 
-WF_KERNEL void k_schedule(Dev d, int force) {
+// rigid: the planes' velocities of the step too (any thread's share)
+WF_KERNEL void k_schedule(Dev d, int force, int rigid, BcTable bc) {
+  if (rigid) rigid_bc(d, bc, blockIdx.x * kBlock + threadIdx.x);
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   DevFlags *f = d.flags;
   const int isfirst = f->step == 0;
@@ -273,7 +305,7 @@ __device__ inline void scan_chunk(const int *cnt, int *loc, int *tot, int ncells
     if (c0 + k < ncells) loc[c0 + k] = off;
     off += v[k];
   }
-  if (threadIdx.x == 0) tot[b] = t;
+  if (threadIdx.x == 0) put_agent(&tot[b], t);
 }
 
 // exclusive scan of the chunk totals written by the other blocks of the
@@ -282,7 +314,7 @@ __device__ inline void scan_totals(const int *tot, int *off, int nch, int *end, 
   int carry = 0;
   for (int base = 0; base < nch; base += kScanThreads) {
     const int q = base + threadIdx.x;
-    const int v = q < nch ? __hip_atomic_load(&tot[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    const int v = q < nch ? get_agent(&tot[q]) : 0;
     int t;
     const int e = block_scan_excl(v, sh, &t);
     if (q < nch) off[q] = carry + e;
@@ -312,18 +344,17 @@ __global__ __launch_bounds__(kScanThreads) void k_scan(Dev d) {
   if (threadIdx.x == 0) {
     unsigned m = 0;
     for (int w = 0; w < kScanThreads / 64; ++w) m = max(m, (unsigned)sh[w]);
-    d.hred[b] = m;
-    __threadfence();
+    put_agent(&d.hred[b], m);
+    stores_done();
     last = atomicAdd(&d.flags->scan_ticket, 1u) == (unsigned)(nb - 1);
   }
   __syncthreads();
   if (!last) return;
-  __threadfence();
   scan_totals(d.ctot, d.coff, ns, d.cell_start + d.sncells, sh);
   if (nr) scan_totals(d.rtot, d.roff, nr, d.rstart + d.ncells, sh);
   hb = 0;
   for (int q = threadIdx.x; q < nb; q += kScanThreads)
-    hb = max(hb, __hip_atomic_load(&d.hred[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    hb = max(hb, get_agent(&d.hred[q]));
   for (int o = 32; o > 0; o >>= 1) hb = max(hb, (unsigned)__shfl_xor((int)hb, o, 64));
   __syncthreads();
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = (int)hb;
@@ -932,8 +963,9 @@ WF_KERNEL void k_plane_strain(Dev d) {
 }
 void launch_plane_strain(const Dev &d, hipStream_t st) { k_plane_strain<<<d.nblocks, kBlock, 0, st>>>(d); }
 
-void launch_schedule(const Dev &d, hipStream_t st, int force) {
-  k_schedule<<<1, 64, 0, st>>>(d, force);
+void launch_schedule(const Dev &d, hipStream_t st, int force, const BcTable *bc) {
+  const int rigid = bc && d.contact;
+  k_schedule<<<rigid ? nblk(d.nrig) : 1, kBlock, 0, st>>>(d, force, rigid, bc ? *bc : BcTable{});
 }
 
 void launch_neighbours(const Dev &d, hipStream_t st, int cur) {
@@ -2985,7 +3017,8 @@ __device__ inline double fin_op(int op, double v, double x) {
   return op == 0 ? v + x : (op == 1 ? fmax(v, x) : fmin(v, x));
 }
 
-__device__ void fin_apply(const Dev &d, double dt, const FinList &L) {
+// val: the reduced slots, in the list's order
+__device__ void fin_apply(const Dev &d, double dt, const FinList &L, const double *val) {
   if (dt < 0) dt = d.flags->dt;
   DevFlags *f = d.flags;
   const long long step = f->step;
@@ -2993,8 +3026,7 @@ __device__ void fin_apply(const Dev &d, double dt, const FinList &L) {
   double e_kin = 0.0, e_int = 0.0, plw = 0.0, tmax = 0.0, tmin = 0.0, cfsum = 0.0, creact = 0.0, extw = 0.0;
   for (int k = 0; k < L.n; ++k) {
     const int s = L.slot[k];
-    // written by the other blocks of this launch: read past the L1 cache
-    const double r = __hip_atomic_load(&d.fin[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const double r = val[k];
     if (s == P_KIN) e_kin = r;
     if (s == P_INT) e_int = r;
     if (s == P_PLW) plw = r;
@@ -3030,10 +3062,69 @@ __device__ void fin_apply(const Dev &d, double dt, const FinList &L) {
   f->time += dt;
 }
 
+// TriMesh::Update of mesh m by one block (Source/Mesh.cpp:273-296): node
+// velocity m_v + m_w x node at the node's position before it moves, nodes
+// move with it, element normals and plane coefficients are recomputed from
+// the winding, particles take the mean node velocity.  drift: the rigid
+// particles' drift with their old velocities first (the reference's loop
+// covers them).
+__device__ inline void mesh_update(const Dev &d, int m, double dt, int drift) {
+  const double4 mv = d.mv[m], mw = d.mw[m];
+  const int n0 = d.mesh_node0[m], nn = d.mesh_nnode[m];
+  for (int k = threadIdx.x; k < nn; k += blockDim.x) {
+    double4 p = d.node[n0 + k];
+    const double wp[3] = {mw.y * p.z - mw.z * p.y, mw.z * p.x - mw.x * p.z, mw.x * p.y - mw.y * p.x};
+    const double4 nv = make_double4(mv.x + wp[0], mv.y + wp[1], mv.z + wp[2], 0.0);
+    p.x += nv.x * dt;
+    p.y += nv.y * dt;
+    p.z += nv.z * dt;
+    d.node[n0 + k] = p;
+    d.nodev[n0 + k] = nv;
+  }
+  __syncthreads();
+  const int e0 = d.mesh_elem0[m], ne = d.mesh_nelem[m];
+  for (int e = threadIdx.x; e < ne; e += blockDim.x) {
+    const int4 el = d.elem[e0 + e];
+    if (drift) {
+      double4 x = d.rx[e0 + e];
+      const double4 v = d.rv[e0 + e];
+      x.x += v.x * dt;
+      x.y += v.y * dt;
+      x.z += v.z * dt;
+      d.rx[e0 + e] = x;
+    }
+    const double4 a = d.node[el.x], b = d.node[el.y], c = d.node[el.z];
+    const double u[3] = {b.x - a.x, b.y - a.y, b.z - a.z}, v[3] = {c.x - a.x, c.y - a.y, c.z - a.z};
+    double w[3];
+    cross_d(u, v, w);
+    const double nw = sqrt(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]);
+    const double n[3] = {w[0] / nw, w[1] / nw, w[2] / nw};
+    const double4 pf = el.w == 0 ? a : (el.w == 1 ? b : c);
+    const double pp = pf.x * n[0] + pf.y * n[1] + pf.z * n[2];
+    d.enorm[e0 + e] = make_double4(n[0], n[1], n[2], pp);
+    const double4 va = d.nodev[el.x], vb = d.nodev[el.y], vc = d.nodev[el.z];
+    const double vm = ((0.0 + va.x) + vb.x) + vc.x;
+    const double vn = ((0.0 + va.y) + vb.y) + vc.y;
+    const double vo = ((0.0 + va.z) + vb.z) + vc.z;
+    d.rv[e0 + e] = make_double4(vm / 3, vn / 3, vo / 3, 0.0);
+  }
+}
+
+// blocks [0, L.n): the slots; then one block per rigid mesh.  The handed-over
+// sums are written through and loaded by as many threads at once: with
+// __threadfence() and one thread loading them in turn the kernel took 6-12 us,
+// 5.8 us at 4.5k particles and 16 with two meshes of 2,048 triangles now; the
+// meshes' update was a launch of its own of 10-15 us and the drift
+// one of 4.6 us.
 constexpr int kFinThreads = 1024;
-__global__ __launch_bounds__(kFinThreads) void k_finalize(Dev d, double dt, FinList L) {
+__global__ __launch_bounds__(kFinThreads) void k_finalize(Dev d, double dt, FinList L, int drift) {
   __shared__ double sh[kFinThreads / 64];
+  __shared__ double val[P_COUNT];
   __shared__ int last;
+  if ((int)blockIdx.x >= L.n) {
+    mesh_update(d, blockIdx.x - L.n, dt < 0 ? d.flags->dt : dt, drift);
+    return;
+  }
   const int s = L.slot[blockIdx.x], op = L.op[blockIdx.x];
   const int nb = d.nblocks;
   double v = op == 0 ? 0.0 : (op == 1 ? -INFINITY : INFINITY);
@@ -3053,18 +3144,20 @@ __global__ __launch_bounds__(kFinThreads) void k_finalize(Dev d, double dt, FinL
   else if (op == 1) r = block_reduce<1>(v, sh);
   else r = block_reduce<2>(v, sh);
   if (threadIdx.x == 0) {
-    d.fin[s] = r;
-    __threadfence();
+    put_agent(&d.fin[s], r);
+    stores_done();
     last = atomicAdd(&d.flags->fin_ticket, 1u) == (unsigned)(L.n - 1);
   }
   __syncthreads();
-  if (!last || threadIdx.x != 0) return;
-  __threadfence();
-  fin_apply(d, dt, L);
+  if (!last) return;
+  if ((int)threadIdx.x < L.n) val[threadIdx.x] = get_agent(&d.fin[L.slot[threadIdx.x]]);
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  fin_apply(d, dt, L, val);
   d.flags->fin_ticket = 0;
 }
 
-void launch_finalize(const Dev &d, hipStream_t st, double dt, int nz) {
+void launch_finalize(const Dev &d, hipStream_t st, double dt, int nz, int drift) {
   FinList L{};
   auto add = [&](int s, int op) {
     L.slot[L.n] = s;
@@ -3089,7 +3182,7 @@ void launch_finalize(const Dev &d, hipStream_t st, double dt, int nz) {
       add(P_CHC, 0);
     }
   }
-  k_finalize<<<L.n, kFinThreads, 0, st>>>(d, dt, L);
+  k_finalize<<<L.n + (d.contact ? d.nmesh : 0), kFinThreads, 0, st>>>(d, dt, L, drift);
 }
 
 // ---------------------------------------------------------------------------
@@ -3189,36 +3282,8 @@ WF_KERNEL void k_surface(Dev d, int cur, int setup) {
   }
 }
 
-// velocity of each plane and of its particles at the step's time
-// (UserAcc's BC loop and the contact-mesh branch, Source/WeldForm.cpp:67-119)
-WF_KERNEL void k_rigid_bc(Dev d, BcTable bc) {
-  const int r = blockIdx.x * kBlock + threadIdx.x;
-  if (r >= d.nrig) return;
-  const int m = d.rmesh[r];
-  const int zone = d.mesh_zone[m];
-  bool set = false, wset = false;
-  double v[3] = {0, 0, 0}, w[3] = {0, 0, 0};
-  for (int b = 0; b < bc.n; ++b) {
-    if (bc.zone[b] != zone || bc.type[b] != 0) continue;
-    if (bc.value_type[b] == 1) {
-      if (bc.amp[b] < 0) continue;
-      const double f = bc.amp_factor[b] * amp_value(d.amps[bc.amp[b]], d.flags->time);
-      for (int k = 0; k < 3; ++k) v[k] = f * bc.v[b][k];
-    } else {
-      for (int k = 0; k < 3; ++k) v[k] = bc.v[b][k];
-      // SetRotAxisVel: constant BCs only (Source/WeldForm.cpp:97-101)
-      for (int k = 0; k < 3; ++k) w[k] = bc.w[b][k];
-      wset = true;
-    }
-    set = true;
-  }
-  if (!set) return;
-  d.rv[r] = make_double4(v[0], v[1], v[2], 0.0);
-  if (r == d.mesh_elem0[m]) {
-    d.mv[m] = make_double4(v[0], v[1], v[2], 0.0);
-    if (wset) d.mw[m] = make_double4(w[0], w[1], w[2], 0.0);
-  }
-}
+// the planes' velocities alone, for a step run in parts
+WF_KERNEL void k_rigid_bc(Dev d, BcTable bc) { rigid_bc(d, bc, blockIdx.x * kBlock + threadIdx.x); }
 
 // Wang contact force of each particle over its partners, in order
 WF_KERNEL void k_contact(Dev d, int cur, double dt) {
@@ -3699,7 +3764,8 @@ void launch_group_sums(const Dev &d, hipStream_t st, int what) {
   if (d.ngroups > 0) k_group_sums<<<d.ngchunks, kGroupThreads, 0, st>>>(d, what);
 }
 
-// the drift of the rigid particles (the reference's loop covers them)
+// the drift of the rigid particles alone, for a step run in parts (a whole
+// step drifts them with the mesh update)
 WF_KERNEL void k_rigid_drift(Dev d, double dt) {
   if (dt < 0) dt = d.flags->dt;
   const int r = blockIdx.x * kBlock + threadIdx.x;
@@ -3712,52 +3778,13 @@ WF_KERNEL void k_rigid_drift(Dev d, double dt) {
   d.rx[r] = x;
 }
 
-// one block per mesh (TriMesh::Update, Source/Mesh.cpp:273-296): node
-// velocity m_v + m_w x node at the node's position before it moves, nodes
-// move with it, element normals and plane coefficients are recomputed from
-// the winding, particles take the mean node velocity
-__global__ __launch_bounds__(1024) void k_mesh_update(Dev d, double dt) {
-  if (dt < 0) dt = d.flags->dt;
-  const int m = blockIdx.x;
-  const double4 mv = d.mv[m], mw = d.mw[m];
-  const int n0 = d.mesh_node0[m], nn = d.mesh_nnode[m];
-  for (int k = threadIdx.x; k < nn; k += blockDim.x) {
-    double4 p = d.node[n0 + k];
-    const double wp[3] = {mw.y * p.z - mw.z * p.y, mw.z * p.x - mw.x * p.z, mw.x * p.y - mw.y * p.x};
-    const double4 nv = make_double4(mv.x + wp[0], mv.y + wp[1], mv.z + wp[2], 0.0);
-    p.x += nv.x * dt;
-    p.y += nv.y * dt;
-    p.z += nv.z * dt;
-    d.node[n0 + k] = p;
-    d.nodev[n0 + k] = nv;
-  }
-  __syncthreads();
-  const int e0 = d.mesh_elem0[m], ne = d.mesh_nelem[m];
-  for (int e = threadIdx.x; e < ne; e += blockDim.x) {
-    const int4 el = d.elem[e0 + e];
-    const double4 a = d.node[el.x], b = d.node[el.y], c = d.node[el.z];
-    const double u[3] = {b.x - a.x, b.y - a.y, b.z - a.z}, v[3] = {c.x - a.x, c.y - a.y, c.z - a.z};
-    double w[3];
-    cross_d(u, v, w);
-    const double nw = sqrt(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]);
-    const double n[3] = {w[0] / nw, w[1] / nw, w[2] / nw};
-    const int fa = el.w == 0 ? el.x : (el.w == 1 ? el.y : el.z);
-    const double4 pf = d.node[fa];
-    const double pp = pf.x * n[0] + pf.y * n[1] + pf.z * n[2];
-    d.enorm[e0 + e] = make_double4(n[0], n[1], n[2], pp);
-    const double4 va = d.nodev[el.x], vb = d.nodev[el.y], vc = d.nodev[el.z];
-    const double vm = ((0.0 + va.x) + vb.x) + vc.x;
-    const double vn = ((0.0 + va.y) + vb.y) + vc.y;
-    const double vo = ((0.0 + va.z) + vb.z) + vc.z;
-    d.rv[e0 + e] = make_double4(vm / 3, vn / 3, vo / 3, 0.0);
-  }
-}
-
 void launch_surface(const Dev &d, hipStream_t st, int cur, int setup) {
   k_surface<<<nblk(d.n), kBlock, 0, st>>>(d, cur, setup);
 }
-void launch_contact(const Dev &d, hipStream_t st, const BcTable &bc, int cur, double dt, int law) {
-  k_rigid_bc<<<(d.nrig + kBlock - 1) / kBlock, kBlock, 0, st>>>(d, bc);
+void launch_rigid_bc(const Dev &d, hipStream_t st, const BcTable &bc) {
+  k_rigid_bc<<<nblk(d.nrig), kBlock, 0, st>>>(d, bc);
+}
+void launch_contact(const Dev &d, hipStream_t st, int cur, double dt, int law) {
   switch (law) {
     case 0: k_contact_law<0><<<d.nblocks, kBlock, 0, st>>>(d, cur, dt); break;
     case 2: k_contact_law<2><<<d.nblocks, kBlock, 0, st>>>(d, cur, dt); break;
@@ -3768,7 +3795,6 @@ void launch_contact(const Dev &d, hipStream_t st, const BcTable &bc, int cur, do
 void launch_rigid_drift(const Dev &d, hipStream_t st, double dt) {
   k_rigid_drift<<<(d.nrig + kBlock - 1) / kBlock, kBlock, 0, st>>>(d, dt);
 }
-void launch_mesh_update(const Dev &d, hipStream_t st, double dt) { k_mesh_update<<<d.nmesh, 1024, 0, st>>>(d, dt); }
 
 // ---------------------------------------------------------------------------
 // utilities
