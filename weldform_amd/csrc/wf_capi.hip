@@ -6,11 +6,14 @@
 // KickDrift loops.  No host<->device synchronisation happens inside
 // wf_step: the neighbour-search schedule lives on the device.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstddef>
 #include <cstring>
 #include <stdexcept>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "wf_internal.h"
@@ -154,6 +157,9 @@ struct Ctx {
   // output staging (wf_pack_*): allocated on first use, not snapshotted
   void *outbuf = nullptr;
   size_t out_cap = 0;
+  // pinned chunks of copy_out, one per thread, allocated on first use
+  std::vector<void *> pin;
+  std::vector<hipEvent_t> pin_ev;
   template <class T>
   T *adj_alloc(size_t count) {
     void *p = nullptr;
@@ -177,6 +183,8 @@ struct Ctx {
     for (auto &p : allocs) (void)hipFree(p.first);
     for (void *p : adj.mem) (void)hipFree(p);
     if (outbuf) (void)hipFree(outbuf);
+    for (void *p : pin) (void)hipHostFree(p);
+    for (auto &e : pin_ev) (void)hipEventDestroy(e);
     if (st) (void)hipStreamDestroy(st);
   }
 };
@@ -1563,6 +1571,60 @@ static void *out_staging(Ctx *c, size_t bytes) {
   return c->outbuf;
 }
 
+// Device table to the caller's (pageable) memory.  The runtime's own pageable
+// copy goes through one staging chunk at a time: 25 ms for the 256 MB of 954k
+// particles.  Here a few threads each bring chunks into a pinned buffer of
+// their own and copy them on while the others' are in flight: 6.9 ms.  Below
+// kCopyMin bytes the threads cost more than they give.  The caller has made
+// the table's kernel the stream's last work; returns when the copy is done.
+constexpr size_t kCopyChunk = (size_t)4 << 20, kCopyMin = (size_t)16 << 20;
+constexpr int kCopyThreads = 8;
+static void copy_out(Ctx *c, void *dst, const void *src, size_t bytes) {
+  const size_t nch = (bytes + kCopyChunk - 1) / kCopyChunk;
+  if (bytes >= kCopyMin)
+    while ((int)c->pin.size() < kCopyThreads) {
+      void *p = nullptr;
+      hipEvent_t e{};
+      if (hipHostMalloc(&p, kCopyChunk, hipHostMallocDefault) != hipSuccess) break;
+      if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+        (void)hipHostFree(p);
+        break;
+      }
+      c->pin.push_back(p);
+      c->pin_ev.push_back(e);
+    }
+  (void)hipGetLastError();  // (without pinned memory the plain copy below does)
+  const int nt = bytes >= kCopyMin ? (int)c->pin.size() : 0;
+  if (nt == 0) {
+    HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipStreamSynchronize(c->st));
+    return;
+  }
+  std::atomic<size_t> next{0};
+  std::atomic<int> err{(int)hipSuccess};
+  auto work = [&](int t) {
+    hipError_t e = hipSetDevice(c->cfg.device);
+    for (size_t k = next++; e == hipSuccess && k < nch; k = next++) {
+      const size_t off = k * kCopyChunk, len = std::min(kCopyChunk, bytes - off);
+      e = hipMemcpyAsync(c->pin[t], (const char *)src + off, len, hipMemcpyDeviceToHost, c->st);
+      if (e == hipSuccess) e = hipEventRecord(c->pin_ev[t], c->st);
+      if (e == hipSuccess) e = hipEventSynchronize(c->pin_ev[t]);
+      if (e == hipSuccess) std::memcpy((char *)dst + off, c->pin[t], len);
+    }
+    if (e != hipSuccess) err = (int)e;
+  };
+  std::vector<std::thread> team;
+  team.reserve(nt);
+  try {
+    for (int t = 1; t < nt; ++t) team.emplace_back(work, t);
+  } catch (const std::system_error &) {
+    // fewer threads: the others take the chunks
+  }
+  work(0);
+  for (std::thread &t : team) t.join();
+  HIPCHK((hipError_t)err.load());
+}
+
 int wf_pack_xdmf(void *ctx, float *f, int32_t *iv) {
   Ctx *c = (Ctx *)ctx;
   return guard(c, [&] {
@@ -1575,9 +1637,8 @@ int wf_pack_xdmf(void *ctx, float *f, int32_t *iv) {
     int *di = (int *)(buf + nf * 4);
     launch_pack_xdmf(c->d, c->st, c->cur, df, di);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(f, df, nf * 4, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipMemcpyAsync(iv, di, ni * 4, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipStreamSynchronize(c->st));
+    copy_out(c, f, df, nf * 4);
+    copy_out(c, iv, di, ni * 4);
     return WF_OK;
   });
 }
@@ -1622,8 +1683,7 @@ int wf_pack_csv(void *ctx, double *rows) {
     double *dr = (double *)out_staging(c, nr * 8);
     launch_pack_csv(c->d, c->st, c->cur, dr);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(rows, dr, nr * 8, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipStreamSynchronize(c->st));
+    copy_out(c, rows, dr, nr * 8);
     return WF_OK;
   });
 }
