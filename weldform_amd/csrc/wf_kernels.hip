@@ -2064,28 +2064,86 @@ void launch_kick(const Dev &d, hipStream_t st, const BcTable &bc, int scheme, do
 // the smallest neighbour distance over CFL (Cs + |v|), or sqrt_h_a
 // sqrt(h / |a|) (the acceleration criterion, evaluated last, wins when both
 // are on); block minima, then AdaptiveTimeStep (:206-239) in one thread.
-WF_KERNEL void k_ts_check(Dev d, int cur) {
+//
+// The distance pass reads FP64 positions from the tile's LDS copy, four lanes
+// per particle (tiles that are not staged: from HBM).  The square root is
+// monotonic, so the least square gives the least distance exactly.  One lane
+// per particle gathering the positions from HBM, a root per neighbour, took
+// 35 us at 35k particles, now 7.2 us.
+struct PosLds {
+  const double2 *xy;
+  const double *z;
+  __device__ double3 load(int p) const { return make_double3(xy[p].x, xy[p].y, z[p]); }
+};
+struct PosHbm {
+  const double4 *x;
+  __device__ double3 load(int j) const {
+    const double4 a = x[j];
+    return make_double3(a.x, a.y, a.z);
+  }
+};
+template <class Rows, class Rec>
+__device__ inline double least_r2(const Rows &rows, const Rec &rec, int own, int cnt, int sub, const double4 &xi,
+                                  typename Rows::G a0, typename Rows::G b0) {
+#pragma clang fp contract(off)
+  double mn = INFINITY;
+  walk_groups<kLanesLds64>(rows, cnt, sub, rows.self(), a0, b0, [&](const typename Rows::G &c) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int p = entry(c, u);
+      const double3 x = rec.load(p);
+      const double dx = x.x - xi.x, dy = x.y - xi.y, dz = x.z - xi.z;
+      const double r2 = dx * dx + dy * dy + dz * dz;
+      mn = fmin(mn, p == own ? INFINITY : r2);  // (padding entries are the particle itself)
+    }
+  });
+  return mn;
+}
+__global__ __launch_bounds__(kBlock *kLanesLds64) void k_ts_vel(Dev d, int cur) {
+#pragma clang fp contract(off)
+  constexpr int NT = kBlock * kLanesLds64;
+  __shared__ double2 xy[kStageMax];
+  __shared__ double z[kStageMax];
+  __shared__ double red[(kLanesLds64 - 1) * kBlock];
+  __shared__ double sh[NT / 64];
+  const int t = xcd_tile(blockIdx.x, gridDim.x), sub = threadIdx.x / kBlock, lane = threadIdx.x % kBlock;
+  const int i = t * kBlock + lane;
+  const int U = d.stage_cnt[t];
+  const int cnt = i < d.n ? d.nnb[i] : 0;
+  const double4 xi = d.xh[cur][i];
+  double mn;
+  if (U < 0) {
+    const HbmRows rows{reinterpret_cast<const int4 *>(d.nbr) + i, d.npad, i};
+    mn = least_r2(rows, PosHbm{d.xh[cur]}, i, cnt, sub, xi, rows.group(2 * sub), rows.group(2 * sub + 1));
+  } else {
+    const LdsRows rows{reinterpret_cast<const ushort4 *>(d.nbrl) + i, d.npad, (int)d.selfl[i]};
+    const ushort4 a0 = rows.group(2 * sub), b0 = rows.group(2 * sub + 1);
+    stage_set<NT>(d, t, U, [&](int p, int j) {
+      const double4 x = d.xh[cur][j];
+      xy[p] = make_double2(x.x, x.y);
+      z[p] = x.z;
+    });
+    mn = least_r2(rows, PosLds{xy, z}, rows.own, cnt, sub, xi, a0, b0);
+  }
+  if (sub > 0) red[(sub - 1) * kBlock + lane] = mn;
+  __syncthreads();
+  double test = INFINITY;
+  if (sub == 0 && i < d.n) {
+    for (int q = 0; q < kLanesLds64 - 1; ++q) mn = fmin(mn, red[q * kBlock + lane]);
+    const double4 v = d.vm[i];
+    test = d.cfl * fmin(1000., sqrt(mn)) / (d.mats[d.mat[i]].Cs + sqrt(v.x * v.x + v.y * v.y + v.z * v.z));
+  }
+  const double r = block_reduce<2>(test, sh);
+  if (threadIdx.x == 0) part(d, P_DTMIN, t) = r;
+}
+WF_KERNEL void k_ts_acc(Dev d, int cur) {
 #pragma clang fp contract(off)
   __shared__ double sh[kBlock / 64];
   const int i = blockIdx.x * kBlock + threadIdx.x;
   double test = INFINITY;
   if (i < d.n) {
-    const double4 xi = d.xh[cur][i];
-    if (d.auto_ts & 2) {
-      const double4 a = d.acc[i];
-      test = d.sqrt_h_a * sqrt(xi.w / sqrt(a.x * a.x + a.y * a.y + a.z * a.z));
-    } else {
-      double mn = 1000.;
-      const int cnt = d.nnb[i];
-      for (int k = 0; k < cnt; ++k) {
-        const double4 xj = d.xh[cur][d.nbr[nb_slot(d.npad, k, i)]];
-        const double dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
-        const double dd = sqrt(dx * dx + dy * dy + dz * dz);
-        if (dd < mn) mn = dd;
-      }
-      const double4 v = d.vm[i];
-      test = d.cfl * mn / (d.mats[d.mat[i]].Cs + sqrt(v.x * v.x + v.y * v.y + v.z * v.z));
-    }
+    const double4 a = d.acc[i];
+    test = d.sqrt_h_a * sqrt(d.xh[cur][i].w / sqrt(a.x * a.x + a.y * a.y + a.z * a.z));
   }
   const double r = block_reduce<2>(test, sh);
   if (threadIdx.x == 0) part(d, P_DTMIN, blockIdx.x) = r;
@@ -2122,7 +2180,8 @@ __global__ __launch_bounds__(1024) void k_ts_adapt(Dev d) {
 }
 
 void launch_time_step(const Dev &d, hipStream_t st, int cur) {
-  k_ts_check<<<d.nblocks, kBlock, 0, st>>>(d, cur);
+  if (d.auto_ts & 2) k_ts_acc<<<d.nblocks, kBlock, 0, st>>>(d, cur);
+  else k_ts_vel<<<d.nblocks, kBlock * kLanesLds64, 0, st>>>(d, cur);
   k_ts_adapt<<<1, 1024, 0, st>>>(d);
 }
 
