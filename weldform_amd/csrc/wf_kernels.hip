@@ -497,9 +497,13 @@ __device__ inline void sort_cell(const Dev &d, int cur, int c, int lane) {
 // larger ones one after another (sort_cell), so grids of mostly empty
 // cells cost little.  The wavefronts, and the threads writing the
 // rigid grid's starts, stride over the cells (a modest grid, so a step
-// without a search exits early at little cost).
-constexpr int kSortGroup = 16;
-WF_KERNEL void k_cell_sort(Dev d, int cur) {
+// without a search exits early at little cost).  A wavefront works through its
+// group's larger cells one after another, so the group is as small as the
+// grid allows (16 cells per wavefront on a grid of 5 thousand took 45 us per
+// search of 35k particles, one 9 us; 3.7k 40 and 7, 370k 55 and 27, 954k 71
+// and 52).
+constexpr int kSortGroup = 16, kSortBlocks = 8192;
+WF_KERNEL void k_cell_sort(Dev d, int cur, int group) {
   if (!d.flags->do_search) return;
   if (d.nrig)
     for (int c = blockIdx.x * kBlock + threadIdx.x; c < d.ncells; c += gridDim.x * kBlock) {
@@ -508,10 +512,10 @@ WF_KERNEL void k_cell_sort(Dev d, int cur) {
     }
   const int lane = threadIdx.x & 63;
   const int nw = gridDim.x * (kBlock / 64);
-  for (int base = (blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * kSortGroup; base < d.sncells;
-       base += nw * kSortGroup) {
+  for (int base = (blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * group; base < d.sncells;
+       base += nw * group) {
     const int c = base + lane;
-    const bool mine = lane < kSortGroup && c < d.sncells;
+    const bool mine = lane < group && c < d.sncells;
     int cnt = 0;
     if (mine) {
       const int s = cell_first(d, c), e = cell_end(d, c);
@@ -696,6 +700,120 @@ WF_KERNEL void k_build_nbr(Dev d, int cur) {
   // deterministic totals via block reduction + integer atomics
   const double bt = block_reduce<0>((double)cnt, sh);
   const double bm = block_reduce<1>((double)cnt, sh);
+  if (threadIdx.x == 0) {
+    atomicAdd((unsigned long long *)&d.flags->directed_pairs, (unsigned long long)bt);
+    atomicMax(&d.flags->max_count, (int)bm);
+  }
+}
+
+// The same rows with kBuildLanes lanes per particle, for models whose lanes of
+// k_build_nbr would leave most of the chip idle: the first nine lanes form the
+// nine columns' ranges together, then the lanes test as many candidates of a
+// column at a time and append them in the records' order by a count of the
+// lanes below.  Per search, one lane against 32 per particle: 58 and 16.5 us at
+// 1.3k particles, 70 and 28 at 3.7k, but 66 and 214 at 35k.
+constexpr int kBuildLanes = 32;
+WF_KERNEL void k_build_nbr_wide(Dev d, int cur) {
+  if (!d.flags->do_search) return;
+  __shared__ double sh[kBlock / 64];
+  const int sl = threadIdx.x & (kBuildLanes - 1), seg = threadIdx.x & 63 & ~(kBuildLanes - 1);
+  const int ps = (int)((blockIdx.x * (long long)kBlock + threadIdx.x) / kBuildLanes);
+  const int i = ps < d.n ? d.sorted[ps] : ps;
+  const long long np = d.npad;
+  const bool on = i < d.n && d.group[i] >= 0;
+  const int ii = on ? i : 0;
+  const int g = d.group[ii];
+  const double4 xi = d.xh[cur][ii];
+  const int c = d.scell[ii];
+  const int nz = d.scellno[2], ny = d.scellno[1], nx = d.scellno[0];
+  const int cz = c % nz, cy = (c / nz) % ny, cx = c / (nz * ny);
+  const float csx = (float)d.scellsize[0], csy = (float)d.scellsize[1], csz = (float)d.scellsize[2];
+  const float oxi = (float)(xi.x - (d.blpf[0] + cx * d.scellsize[0]));
+  const float oyi = (float)(xi.y - (d.blpf[1] + cy * d.scellsize[1]));
+  const float ozi = (float)(xi.z - (d.blpf[2] + cz * d.scellsize[2]));
+  const float hi = (float)xi.w, hcf = 0.5f * (float)d.cellfac;
+  const bool exact_all = fabsf(oxi) > 64.f * csx || fabsf(oyi) > 64.f * csy || fabsf(ozi) > 64.f * csz;
+  const int az0 = cz > 0 ? cz - 1 : 0, az1 = cz + 1 < nz ? cz + 1 : nz - 1, m = az1 - az0;
+  const float ri = hcf * (hi + __uint_as_float(d.flags->hmax_bits)) * 1.0001f, ri2 = ri * ri;
+  const float inv_hz = 4.f / csz;
+  const int gmax = 4 * m + 3;
+  const float bz0 = (float)(cz - az0) * csz + ozi, bz1 = (float)(cz - az0 - 1) * csz + ozi,
+              bz2 = (float)(cz - az0 - 2) * csz + ozi;
+  // lane col < 9 of the particle: the column's records within reach (see
+  // k_build_nbr), where its cells start and its offset from the particle
+  int lo = 0, hi_end = 0, s1 = 0, s2 = 0;
+  float bx = 0.f, by = 0.f;
+  if (on && sl < 9) {
+    const int dcx = sl / 3 - 1, dcy = sl % 3 - 1;
+    const int ax = cx + dcx, ay = cy + dcy;
+    if (ax >= 0 && ax < nx && ay >= 0 && ay < ny) {
+      bx = (float)(cx - ax) * csx + oxi;
+      by = (float)(cy - ay) * csy + oyi;
+      const int cc0 = (ax * ny + ay) * nz + az0;
+      const int s0 = d.cell_start[cc0];
+      s1 = d.cell_start[cc0 + 1];
+      s2 = m >= 1 ? d.cell_start[cc0 + 2] : s1;
+      lo = s0;
+      hi_end = d.cell_start[cc0 + m + 1];
+      if (!exact_all) {
+        const float gx = fmaxf(dcx < 0 ? oxi : (dcx > 0 ? csx - oxi : 0.f), 0.f);
+        const float gy = fmaxf(dcy < 0 ? oyi : (dcy > 0 ? csy - oyi : 0.f), 0.f);
+        const float rho2 = gx * gx + gy * gy;
+        if (rho2 > ri2) {
+          hi_end = lo;
+        } else {
+          const float w = sqrtf(ri2 - rho2);
+          const int glo = min(max((int)floorf((bz0 - w) * inv_hz), 0), gmax);
+          const int ghi = min(max((int)floorf((bz0 + w) * inv_hz), 0), gmax);
+          const int alo = glo >> 2, klo = glo & 3, ahi = ghi >> 2, khi = ghi & 3;
+          const int4 ol = d.soff[cc0 + alo], oh = d.soff[cc0 + ahi];
+          lo = klo == 0 ? (alo == 0 ? s0 : (alo == 1 ? s1 : s2)) : (klo == 1 ? ol.x : (klo == 2 ? ol.y : ol.z));
+          hi_end = khi == 3 ? oh.w : (khi == 0 ? oh.x : (khi == 1 ? oh.y : oh.z));
+        }
+      }
+    }
+  }
+  int cnt = 0;
+  for (int col = 0; col < 9; ++col) {
+    const int p0 = __shfl(lo, seg + col, 64), p1 = __shfl(hi_end, seg + col, 64);
+    const int q1 = __shfl(s1, seg + col, 64), q2 = __shfl(s2, seg + col, 64);
+    const float cbx = __shfl(bx, seg + col, 64), cby = __shfl(by, seg + col, 64);
+    // (the particles of a wavefront go round together)
+    for (int base = 0; __any(p0 + base < p1); base += kBuildLanes) {
+      const int p = p0 + base + sl;
+      bool in = false;
+      int j = 0;
+      if (p < p1) {
+        const int2 f = d.sinfo[p];
+        const float4 q = d.sxyz[p];
+        j = f.x;
+        const float bz = p >= q2 ? bz2 : (p >= q1 ? bz1 : bz0);
+        const float dx = cbx - q.x, dy = cby - q.y, dz = bz - q.z;
+        const float r2 = dx * dx + dy * dy + dz * dz;
+        const float t = hcf * (hi + q.w);
+        const float t2 = t * t;
+        const bool valid = (j != i) & (f.y == g);
+        in = valid & (r2 < t2);
+        if (valid & (exact_all | (fabsf(r2 - t2) <= 1e-4f * t2))) in = in_radius(xi, d.xh[cur][j], d.cellfac);
+      }
+      const unsigned mask = (unsigned)(__ballot(in) >> seg);
+      const int k = cnt + __popc(mask & ((1u << sl) - 1u));
+      if (in && k < d.max_nb) d.nbr[nb_slot(np, k, i)] = j;
+      cnt += __popc(mask);
+    }
+  }
+  if (i < d.n) {
+    const int kept = cnt < d.max_nb ? cnt : d.max_nb;
+    // the rest of the last group of four holds the particle itself
+    if (sl < ((4 - (kept & 3)) & 3)) d.nbr[nb_slot(np, kept + sl, i)] = i;
+    if (sl == 0) {
+      d.nnb[i] = kept;
+      if (cnt > d.max_nb) d.flags->overflow = 1;
+    }
+  }
+  const double own = sl == 0 ? (double)cnt : 0.0;
+  const double bt = block_reduce<0>(own, sh);
+  const double bm = block_reduce<1>(own, sh);
   if (threadIdx.x == 0) {
     atomicAdd((unsigned long long *)&d.flags->directed_pairs, (unsigned long long)bt);
     atomicMax(&d.flags->max_count, (int)bm);
@@ -968,6 +1086,8 @@ void launch_schedule(const Dev &d, hipStream_t st, int force, const BcTable *bc)
   k_schedule<<<rigid ? nblk(d.nrig) : 1, kBlock, 0, st>>>(d, force, rigid, bc ? *bc : BcTable{});
 }
 
+// rows built with kBuildLanes lanes per particle up to this many particles
+constexpr int kBuildWide = 8192;
 void launch_neighbours(const Dev &d, hipStream_t st, int cur) {
   k_cell_hist<<<nblk((long long)d.n + d.nrig), kBlock, 0, st>>>(d, cur);
   k_scan<<<scan_chunks(d.sncells) + (d.nrig ? scan_chunks(d.ncells) : 0), kScanThreads, 0, st>>>(d);
@@ -976,10 +1096,14 @@ void launch_neighbours(const Dev &d, hipStream_t st, int cur) {
   // as the other search kernels', and 16k wavefronts keep the cells' loads
   // in flight)
   {
-    const int g = nblk((long long)(d.sncells + kSortGroup - 1) / kSortGroup * 64);
-    k_cell_sort<<<g < 8192 ? g : 8192, kBlock, 0, st>>>(d, cur);
+    const int waves = kSortBlocks * (kBlock / 64);
+    int group = (d.sncells + waves - 1) / waves;
+    group = group < kSortGroup ? group : kSortGroup;
+    const int g = nblk((long long)(d.sncells + group - 1) / group * 64);
+    k_cell_sort<<<g < kSortBlocks ? g : kSortBlocks, kBlock, 0, st>>>(d, cur, group);
   }
-  k_build_nbr<<<nblk(d.n), kBlock, 0, st>>>(d, cur);
+  if (d.n <= kBuildWide) k_build_nbr_wide<<<nblk((long long)d.n * kBuildLanes), kBlock, 0, st>>>(d, cur);
+  else k_build_nbr<<<nblk(d.n), kBlock, 0, st>>>(d, cur);
   if (d.stage_max > 0) k_stage<<<d.ntiles < 2048 ? d.ntiles : 2048, kStageThreads, 0, st>>>(d);
 }
 
