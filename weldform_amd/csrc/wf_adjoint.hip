@@ -23,6 +23,8 @@
 // (m_j abar_i - m_i abar_j for the acceleration, vol_j sbar_i + vol_i sbar_j
 // for the density and rate sums), so every particle accumulates its own
 // adjoint in registers: no atomics, deterministic.
+#include <float.h>
+
 #include "wf_device.h"
 
 namespace wf {
@@ -40,6 +42,19 @@ __device__ inline double gk_dr2(double r2, const KH<double> &k) {
     return 0.75 * k.c5 * k.h * ri * ri * (t * k.ih + 0.5 * t * t * ri);
   }
   return 0.0;
+}
+
+// GK and d GK / d r2 together, without branches (r2 = 0, a padding entry of the
+// particle itself: every pair term it enters is an exact zero)
+__device__ inline void gk_both(double r2, const GkD &k, double &GK, double &dGK) {
+  const double ri = rsqrt3(fmax(r2, DBL_MIN));
+  const double q = (r2 * ri) * k.ih;
+  const double t = fmax(2.0 - q, 0.0);
+  const double o = (t * t) * (ri * k.gout);
+  const bool in = q < 1.0;
+  GK = in ? fma(q, k.gin_a, k.gin_b) : o;
+  // inside: 2.25 c5 ih / (2 r); outside: -gout / r^2 (t ih + t^2 / (2 r))
+  dGK = in ? (0.5 * k.gin_a * k.ih) * ri : -(k.gout * ri) * ri * (t * k.ih + (0.5 * t * t) * ri);
 }
 
 // ---------------------------------------------------------------------------
@@ -206,8 +221,63 @@ __device__ inline void rate_seeds(const AdjBufs &b, int j, double sb[6], double 
 // x', v', rho', then the drift x' = x + v' dt and the density update
 // rho' = rho (1 + dt D) backwards
 
-// LANES threads per particle take alternate row entries; their partial
-// sums are added in lane order
+// one pair: e = x_ij, the neighbour's velocity, m/rho and seeds, GK and its
+// derivative by r^2; acc = (xb[3], vb[3], volb)
+__device__ inline void adj_rates_pair(const double3 &e3, const double4 &vi, const double3 &uj, double voli, double volj,
+                                      const double (&sbi)[6], const double (&wbi)[3], const double (&sbj)[6],
+                                      const double (&wbj)[3], double GK, double dGK, double (&acc)[7]) {
+  const double dx = e3.x, dy = e3.y, dz = e3.z;
+  const double vx = vi.x - uj.x, vy = vi.y - uj.y, vz = vi.z - uj.z;
+  const double cp = -0.5 * GK;
+  const double e[6] = {2 * vx * dx, 2 * vy * dy, 2 * vz * dz, vx * dy + vy * dx, vx * dz + vz * dx, vy * dz + vz * dy};
+  const double w[3] = {vx * dy - vy * dx, vx * dz - vz * dx, vy * dz - vz * dy};
+  double eb[6], wbv[3], cpb = 0.0;
+  for (int k = 0; k < 6; ++k) {
+    eb[k] = volj * sbi[k] + voli * sbj[k];
+    cpb += eb[k] * e[k];
+    acc[6] += sbj[k] * cp * e[k];
+  }
+  for (int k = 0; k < 3; ++k) {
+    wbv[k] = volj * wbi[k] + voli * wbj[k];
+    cpb += wbv[k] * w[k];
+    acc[6] += wbj[k] * cp * w[k];
+  }
+  for (int k = 0; k < 6; ++k) eb[k] *= cp;
+  for (int k = 0; k < 3; ++k) wbv[k] *= cp;
+  double bvx = 2 * eb[0] * dx + eb[3] * dy + eb[4] * dz + wbv[0] * dy + wbv[1] * dz;
+  double bvy = 2 * eb[1] * dy + eb[3] * dx + eb[5] * dz - wbv[0] * dx + wbv[2] * dz;
+  double bvz = 2 * eb[2] * dz + eb[4] * dx + eb[5] * dy - wbv[1] * dx - wbv[2] * dy;
+  double bdx = 2 * eb[0] * vx + eb[3] * vy + eb[4] * vz - wbv[0] * vy - wbv[1] * vz;
+  double bdy = 2 * eb[1] * vy + eb[3] * vx + eb[5] * vz + wbv[0] * vx - wbv[2] * vz;
+  double bdz = 2 * eb[2] * vz + eb[4] * vx + eb[5] * vy + wbv[1] * vx + wbv[2] * vy;
+  const double r2b = -0.5 * cpb * dGK;
+  bdx += 2 * r2b * dx;
+  bdy += 2 * r2b * dy;
+  bdz += 2 * r2b * dz;
+  acc[3] += bvx, acc[4] += bvy, acc[5] += bvz;
+  acc[0] += bdx, acc[1] += bdy, acc[2] += bdz;
+}
+// the particle's end of the pass: x' and v' adjoints, then the drift and the
+// density update
+__device__ inline void adj_rates_own(const Dev &d, const AdjSlot &s0, const AdjBufs &b, double dt, int i,
+                                     const double4 &vi, double rhoi1, const double (&acc)[7]) {
+  const double xb[3] = {acc[0], acc[1], acc[2]}, vb[3] = {acc[3], acc[4], acc[5]}, volb = acc[6];
+  // x' and v' adjoints: incoming state adjoint plus the gather
+  const double4 xin = b.xb[i], vin = b.vb[i];
+  const double xpb[3] = {xin.x + xb[0], xin.y + xb[1], xin.z + xb[2]};
+  const double rho0 = s0.rho[i];
+  const double rhopb = b.rhob[i] + volb * (-vi.w / (rhoi1 * rhoi1));
+  // drift: x' = x + v' dt
+  b.xb[i] = make_double4(xpb[0], xpb[1], xpb[2], 0.0);
+  b.vpb[i] = make_double4(vin.x + vb[0] + dt * xpb[0], vin.y + vb[1] + dt * xpb[1], vin.z + vb[2] + dt * xpb[2], 0.0);
+  // density update: rho' = rho + dt (D rho), D = drho / rho
+  const double D = s0.drho[i] / rho0;
+  b.rhob[i] = rhopb * (1.0 + dt * D);
+  b.db[i] = rhopb * dt * rho0;
+}
+
+// gathers from HBM: LANES threads per particle take alternate row entries;
+// their partial sums are added in lane order
 template <int LANES>
 __global__ __launch_bounds__(kBlock *LANES) void k_adj_rates(Dev d, AdjSlot s0, AdjSlot s1, AdjBufs b, double dt) {
   __shared__ double red[(LANES > 1 ? LANES - 1 : 1) * 7 * kBlock];
@@ -234,52 +304,85 @@ __global__ __launch_bounds__(kBlock *LANES) void k_adj_rates(Dev d, AdjSlot s0, 
       const double dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
       const double r2 = dx * dx + dy * dy + dz * dz;
       const double GK = gk_t<double>(r2, kh);
-      const double vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
-      const double cp = -0.5 * GK;
-      const double e[6] = {2 * vx * dx, 2 * vy * dy, 2 * vz * dz, vx * dy + vy * dx, vx * dz + vz * dx, vy * dz + vz * dy};
-      const double w[3] = {vx * dy - vy * dx, vx * dz - vz * dx, vy * dz - vz * dy};
-      double eb[6], wbv[3], cpb = 0.0;
-      for (int k = 0; k < 6; ++k) {
-        eb[k] = volj * sbi[k] + voli * sbj[k];
-        cpb += eb[k] * e[k];
-        acc[6] += sbj[k] * cp * e[k];
-      }
-      for (int k = 0; k < 3; ++k) {
-        wbv[k] = volj * wbi[k] + voli * wbj[k];
-        cpb += wbv[k] * w[k];
-        acc[6] += wbj[k] * cp * w[k];
-      }
-      for (int k = 0; k < 6; ++k) eb[k] *= cp;
-      for (int k = 0; k < 3; ++k) wbv[k] *= cp;
-      double bvx = 2 * eb[0] * dx + eb[3] * dy + eb[4] * dz + wbv[0] * dy + wbv[1] * dz;
-      double bvy = 2 * eb[1] * dy + eb[3] * dx + eb[5] * dz - wbv[0] * dx + wbv[2] * dz;
-      double bvz = 2 * eb[2] * dz + eb[4] * dx + eb[5] * dy - wbv[1] * dx - wbv[2] * dy;
-      double bdx = 2 * eb[0] * vx + eb[3] * vy + eb[4] * vz - wbv[0] * vy - wbv[1] * vz;
-      double bdy = 2 * eb[1] * vy + eb[3] * vx + eb[5] * vz + wbv[0] * vx - wbv[2] * vz;
-      double bdz = 2 * eb[2] * vz + eb[4] * vx + eb[5] * vy + wbv[1] * vx + wbv[2] * vy;
-      const double r2b = -0.5 * cpb * gk_dr2(r2, kh);
-      bdx += 2 * r2b * dx;
-      bdy += 2 * r2b * dy;
-      bdz += 2 * r2b * dz;
-      acc[3] += bvx, acc[4] += bvy, acc[5] += bvz;
-      acc[0] += bdx, acc[1] += bdy, acc[2] += bdz;
+      adj_rates_pair(make_double3(dx, dy, dz), vi, make_double3(vj.x, vj.y, vj.z), voli, volj, sbi, wbi, sbj, wbj, GK,
+                     gk_dr2(r2, kh), acc);
     }
   }
   combine_lanes<LANES>(acc, red);
   if (!on || sub != 0) return;
-  const double xb[3] = {acc[0], acc[1], acc[2]}, vb[3] = {acc[3], acc[4], acc[5]}, volb = acc[6];
-  // x' and v' adjoints: incoming state adjoint plus the gather
-  const double4 xin = b.xb[i], vin = b.vb[i];
-  const double xpb[3] = {xin.x + xb[0], xin.y + xb[1], xin.z + xb[2]};
-  const double rho0 = s0.rho[i];
-  const double rhopb = b.rhob[i] + volb * (-vi.w / (rhoi1 * rhoi1));
-  // drift: x' = x + v' dt
-  b.xb[i] = make_double4(xpb[0], xpb[1], xpb[2], 0.0);
-  b.vpb[i] = make_double4(vin.x + vb[0] + dt * xpb[0], vin.y + vb[1] + dt * xpb[1], vin.z + vb[2] + dt * xpb[2], 0.0);
-  // density update: rho' = rho + dt (D rho), D = drho / rho
-  const double D = s0.drho[i] / rho0;
-  b.rhob[i] = rhopb * (1.0 + dt * D);
-  b.db[i] = rhopb * dt * rho0;
+  adj_rates_own(d, s0, b, dt, i, vi, rhoi1, acc);
+}
+
+// From the tile's LDS copy (uniform smoothing lengths): 128 bytes per staged
+// particle, one block per CU, the walk of the forward passes.  At 193k
+// particles the gathers took 196 us (this pass) and 182 us (acceleration),
+// bound by L1 and L2 traffic; from LDS 118 and 143 us.  The entries of a group
+// are not unrolled: four at once need over 256 registers and spill (357 and
+// 355 us).
+__global__ __launch_bounds__(kBlock *kLanesLds64) void k_adj_rates_lds(Dev d, AdjSlot s0, AdjSlot s1, AdjBufs b,
+                                                                       double dt) {
+  constexpr int NT = kBlock * kLanesLds64;
+  __shared__ double2 r[8 * kStageMax];
+  __shared__ double red[(kLanesLds64 - 1) * 7 * kBlock];
+  const int t = xcd_tile(blockIdx.x, gridDim.x), sub = threadIdx.x / kBlock;
+  const int i = t * kBlock + (int)(threadIdx.x % kBlock);
+  const int U = s0.stage_cnt[t];
+  const bool on = i < d.n;
+  const int cnt = on && d.group[i] >= 0 ? s0.nnb[i] : 0;
+  const double4 xi = s1.xh[i], vi = s1.vm[i];
+  const double rhoi1 = on ? s1.rho[i] : 1.0;
+  const double voli = vi.w / rhoi1;
+  double sbi[6], wbi[3];
+  rate_seeds(b, on ? i : 0, sbi, wbi);
+  const GkD k = gk_consts64(xi.w, 3);
+  double acc[7] = {0, 0, 0, 0, 0, 0, 0};
+  auto pair = [&](const double3 &x, const double3 &u, double vol, const double (&sbj)[6], const double (&wbj)[3]) {
+    const double3 e = make_double3(xi.x - x.x, xi.y - x.y, xi.z - x.z);
+    double GK, dGK;
+    gk_both(e.x * e.x + e.y * e.y + e.z * e.z, k, GK, dGK);
+    adj_rates_pair(e, vi, u, voli, vol, sbi, wbi, sbj, wbj, GK, dGK, acc);
+  };
+  if (U < 0) {
+    const HbmRows rows{reinterpret_cast<const int4 *>(s0.nbr) + i, d.npad, i};
+    walk_groups<kLanesLds64>(rows, cnt, sub, rows.self(), rows.group(2 * sub), rows.group(2 * sub + 1), [&](const int4 &c) {
+#pragma unroll 1
+      for (int q = 0; q < 4; ++q) {
+        const int j = entry(c, q);
+        const double4 x = s1.xh[j], v = s1.vm[j];
+        double sbj[6], wbj[3];
+        rate_seeds(b, j, sbj, wbj);
+        pair(make_double3(x.x, x.y, x.z), make_double3(v.x, v.y, v.z), v.w / s1.rho[j], sbj, wbj);
+      }
+    });
+  } else {
+    const LdsRows rows{reinterpret_cast<const ushort4 *>(s0.nbrl) + i, d.npad, (int)s0.selfl[i]};
+    const ushort4 a0 = rows.group(2 * sub), b0 = rows.group(2 * sub + 1);
+    stage_set<NT>(s0.stage, t, U, [&](int p, int j) {
+      const double4 x = s1.xh[j], v = s1.vm[j], a = b.rsb[3 * j], c = b.rsb[3 * j + 1];
+      const double w12 = b.rsb[3 * j + 2].x;
+      r[p] = make_double2(x.x, x.y);
+      r[kStageMax + p] = make_double2(x.z, v.w / s1.rho[j]);
+      r[2 * kStageMax + p] = make_double2(v.x, v.y);
+      r[3 * kStageMax + p] = make_double2(v.z, w12);
+      r[4 * kStageMax + p] = make_double2(a.x, a.y);
+      r[5 * kStageMax + p] = make_double2(a.z, a.w);
+      r[6 * kStageMax + p] = make_double2(c.x, c.y);
+      r[7 * kStageMax + p] = make_double2(c.z, c.w);
+    });
+    walk_groups<kLanesLds64>(rows, cnt, sub, rows.self(), a0, b0, [&](const ushort4 &c) {
+#pragma unroll 1
+      for (int q = 0; q < 4; ++q) {
+        const int p = entry(c, q);
+        const double2 x = r[p], z = r[kStageMax + p], u = r[2 * kStageMax + p], w = r[3 * kStageMax + p];
+        const double2 e0 = r[4 * kStageMax + p], e1 = r[5 * kStageMax + p], e2 = r[6 * kStageMax + p],
+                      e3 = r[7 * kStageMax + p];
+        const double sbj[6] = {e0.x, e0.y, e1.x, e1.y, e2.x, e2.y}, wbj[3] = {e3.x, e3.y, w.y};
+        pair(make_double3(x.x, x.y, z.x), make_double3(u.x, u.y, w.x), z.y, sbj, wbj);
+      }
+    });
+  }
+  combine_lanes<kLanesLds64>(acc, red);
+  if (on && sub == 0) adj_rates_own(d, s0, b, dt, i, vi, rhoi1, acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -525,73 +628,64 @@ __device__ inline void sigma_t(const AdjBufs &b, int j, double t[6], double &rho
   irho2 = c.w;
 }
 
-template <int LANES>
-__global__ __launch_bounds__(kBlock *LANES) void k_adj_accel(Dev d, AdjSlot s0, AdjBufs b) {
-  __shared__ double red[(LANES > 1 ? LANES - 1 : 1) * 13 * kBlock];
-  const int sub = threadIdx.x / kBlock;
-  const int i = blockIdx.x * kBlock + (int)(threadIdx.x % kBlock);
-  const bool on = i < d.n && d.group[i] >= 0;
-  const long long np = d.npad;
-  const DevMat &M = d.mats[on ? d.mat[i] : 0];
-  const double beta = M.beta, acs = M.alpha * M.Cs;
-  const bool av = (M.alpha != 0.0 || M.beta != 0.0);
-  double acc[13] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};  // xb[3], vb[3], tb[6], rhob
-  double ti[6] = {0, 0, 0, 0, 0, 0}, rhoi = 1.0, irho2i = 1.0;
-  if (on) {
-    const double4 xi = s0.xh[i], vi = s0.vm[i], abi = b.ab[i];
-    sigma_t(b, i, ti, rhoi, irho2i);
-    const KH<double> ki = kern_h_t<double>(xi.w);
-    const int cnt = s0.nnb[i];
-    for (int q = sub; q < cnt; q += LANES) {
-      const int j = s0.nbr[nb_slot(np, q, i)];
-      const double4 xj = s0.xh[j], vj = s0.vm[j], abj = b.ab[j];
-      double tj[6], rhoj, irho2j;
-      sigma_t(b, j, tj, rhoj, irho2j);
-      const KH<double> kh = pair_h_t<double>(ki, xi.w, xj.w);
-      const double dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-      const double r2 = dx * dx + dy * dy + dz * dz;
-      const double GK = gk_t<double>(r2, kh);
-      const double vx = vi.x - vj.x, vy = vi.y - vj.y, vz = vi.z - vj.z;
-      const double vdot = vx * dx + vy * dy + vz * dz;
-      const double D1 = r2 + 0.01 * kh.h * kh.h, D2 = 0.5 * (rhoi + rhoj);
-      const double hv = kh.h * vdot / (D1 * D2);
-      const double pv = hv * (acs + beta * (hv * D2));
-      const bool act = av && vdot < 0.0;
-      const double pi = act ? pv : 0.0;
-      const double Mxx = ti[XX] + tj[XX] + pi, Myy = ti[YY] + tj[YY] + pi, Mzz = ti[ZZ] + tj[ZZ] + pi;
-      const double Mxy = ti[XY] + tj[XY], Mxz = ti[XZ] + tj[XZ], Myz = ti[YZ] + tj[YZ];
-      // combined seed of the pair term P_ij = GK M x_ij (a_i += m_j P, a_j -= m_i P)
-      const double cx = vj.w * abi.x - vi.w * abj.x, cy = vj.w * abi.y - vi.w * abj.y,
-                   cz = vj.w * abi.z - vi.w * abj.z;
-      const double mdx = Mxx * dx + Mxy * dy + Mxz * dz, mdy = Mxy * dx + Myy * dy + Myz * dz,
-                   mdz = Mxz * dx + Myz * dy + Mzz * dz;
-      const double GKb = cx * mdx + cy * mdy + cz * mdz;
-      const double mb[6] = {GK * cx * dx, GK * cy * dy, GK * cz * dz, GK * (cx * dy + cy * dx), GK * (cx * dz + cz * dx),
-                            GK * (cy * dz + cz * dy)};
-      for (int k = 0; k < 6; ++k) acc[6 + k] += mb[k];
-      double bdx = GK * (Mxx * cx + Mxy * cy + Mxz * cz);
-      double bdy = GK * (Mxy * cx + Myy * cy + Myz * cz);
-      double bdz = GK * (Mxz * cx + Myz * cy + Mzz * cz);
-      double r2b = GKb * gk_dr2(r2, kh);
-      if (act) {
-        const double pib = mb[0] + mb[1] + mb[2];
-        const double hvb = pib * (acs + 2.0 * beta * hv * D2);
-        double D2b = pib * beta * hv * hv;
-        const double vdb = hvb * kh.h / (D1 * D2);
-        const double D1b = -hvb * hv / D1;
-        D2b += -hvb * hv / D2;
-        r2b += D1b;
-        acc[12] += 0.5 * D2b;
-        acc[3] += vdb * dx, acc[4] += vdb * dy, acc[5] += vdb * dz;
-        bdx += vdb * vx, bdy += vdb * vy, bdz += vdb * vz;
-      }
-      acc[0] += bdx + 2 * r2b * dx;
-      acc[1] += bdy + 2 * r2b * dy;
-      acc[2] += bdz + 2 * r2b * dz;
-    }
+// the particle's side of an acceleration pair
+struct AdjAccOwn {
+  double4 vi, abi;
+  double ti[6], rhoi, acs, beta;
+  bool av;
+};
+// one pair, as adj_rates_pair: the neighbour's velocity and mass, acceleration
+// adjoint, sigma / rho^2 and rho; acc = (xb[3], vb[3], tb[6], rhob)
+__device__ inline void adj_accel_pair(const AdjAccOwn &o, const double3 &e3, double r2, double h, const double3 &uj,
+                                      double mj, const double3 &abj, const double (&tj)[6], double rhoj, double GK,
+                                      double dGK, double (&acc)[13]) {
+  const double dx = e3.x, dy = e3.y, dz = e3.z;
+  const double4 &vi = o.vi, &abi = o.abi;
+  const double (&ti)[6] = o.ti;
+  const double rhoi = o.rhoi, acs = o.acs, beta = o.beta;
+  const bool av = o.av;
+  const double vx = vi.x - uj.x, vy = vi.y - uj.y, vz = vi.z - uj.z;
+  const double vdot = vx * dx + vy * dy + vz * dz;
+  const double D1 = r2 + 0.01 * h * h, D2 = 0.5 * (rhoi + rhoj);
+  const double hv = h * vdot / (D1 * D2);
+  const double pv = hv * (acs + beta * (hv * D2));
+  const bool act = av && vdot < 0.0;
+  const double pi = act ? pv : 0.0;
+  const double Mxx = ti[XX] + tj[XX] + pi, Myy = ti[YY] + tj[YY] + pi, Mzz = ti[ZZ] + tj[ZZ] + pi;
+  const double Mxy = ti[XY] + tj[XY], Mxz = ti[XZ] + tj[XZ], Myz = ti[YZ] + tj[YZ];
+  // combined seed of the pair term P_ij = GK M x_ij (a_i += m_j P, a_j -= m_i P)
+  const double cx = mj * abi.x - vi.w * abj.x, cy = mj * abi.y - vi.w * abj.y,
+               cz = mj * abi.z - vi.w * abj.z;
+  const double mdx = Mxx * dx + Mxy * dy + Mxz * dz, mdy = Mxy * dx + Myy * dy + Myz * dz,
+               mdz = Mxz * dx + Myz * dy + Mzz * dz;
+  const double GKb = cx * mdx + cy * mdy + cz * mdz;
+  const double mb[6] = {GK * cx * dx, GK * cy * dy, GK * cz * dz, GK * (cx * dy + cy * dx), GK * (cx * dz + cz * dx),
+                        GK * (cy * dz + cz * dy)};
+  for (int k = 0; k < 6; ++k) acc[6 + k] += mb[k];
+  double bdx = GK * (Mxx * cx + Mxy * cy + Mxz * cz);
+  double bdy = GK * (Mxy * cx + Myy * cy + Myz * cz);
+  double bdz = GK * (Mxz * cx + Myz * cy + Mzz * cz);
+  double r2b = GKb * dGK;
+  if (act) {
+    const double pib = mb[0] + mb[1] + mb[2];
+    const double hvb = pib * (acs + 2.0 * beta * hv * D2);
+    double D2b = pib * beta * hv * hv;
+    const double vdb = hvb * h / (D1 * D2);
+    const double D1b = -hvb * hv / D1;
+    D2b += -hvb * hv / D2;
+    r2b += D1b;
+    acc[12] += 0.5 * D2b;
+    acc[3] += vdb * dx, acc[4] += vdb * dy, acc[5] += vdb * dz;
+    bdx += vdb * vx, bdy += vdb * vy, bdz += vdb * vz;
   }
-  combine_lanes<LANES>(acc, red);
-  if (!on || sub != 0) return;
+  acc[0] += bdx + 2 * r2b * dx;
+  acc[1] += bdy + 2 * r2b * dy;
+  acc[2] += bdz + 2 * r2b * dz;
+}
+// the particle's end of the pass: t = sigma / rho^2, sigma = S - P(rho) I
+__device__ inline void adj_accel_own(const Dev &d, const AdjBufs &b, int i, const DevMat &M, const double (&ti)[6],
+                                     double rhoi, double irho2i, const double (&acc)[13]) {
+  const long long np = d.npad;
   const double *tb = acc + 6;
   double rhob = acc[12];
   // t = sigma / rho^2, sigma = S - P(rho) I
@@ -609,16 +703,125 @@ __global__ __launch_bounds__(kBlock *LANES) void k_adj_accel(Dev d, AdjSlot s0, 
   b.vb[i] = make_double4(vo.x + acc[3], vo.y + acc[4], vo.z + acc[5], 0.0);
 }
 
+template <int LANES>
+__global__ __launch_bounds__(kBlock *LANES) void k_adj_accel(Dev d, AdjSlot s0, AdjBufs b) {
+  __shared__ double red[(LANES > 1 ? LANES - 1 : 1) * 13 * kBlock];
+  const int sub = threadIdx.x / kBlock;
+  const int i = blockIdx.x * kBlock + (int)(threadIdx.x % kBlock);
+  const bool on = i < d.n && d.group[i] >= 0;
+  const long long np = d.npad;
+  const DevMat &M = d.mats[on ? d.mat[i] : 0];
+  double acc[13] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};  // xb[3], vb[3], tb[6], rhob
+  AdjAccOwn o{};
+  o.rhoi = 1.0, o.acs = M.alpha * M.Cs, o.beta = M.beta, o.av = M.alpha != 0.0 || M.beta != 0.0;
+  double irho2i = 1.0;
+  if (on) {
+    const double4 xi = s0.xh[i];
+    o.vi = s0.vm[i], o.abi = b.ab[i];
+    sigma_t(b, i, o.ti, o.rhoi, irho2i);
+    const KH<double> ki = kern_h_t<double>(xi.w);
+    const int cnt = s0.nnb[i];
+    for (int q = sub; q < cnt; q += LANES) {
+      const int j = s0.nbr[nb_slot(np, q, i)];
+      const double4 xj = s0.xh[j], vj = s0.vm[j], abj = b.ab[j];
+      double tj[6], rhoj, irho2j;
+      sigma_t(b, j, tj, rhoj, irho2j);
+      const KH<double> kh = pair_h_t<double>(ki, xi.w, xj.w);
+      const double3 e = make_double3(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z);
+      const double r2 = e.x * e.x + e.y * e.y + e.z * e.z;
+      adj_accel_pair(o, e, r2, kh.h, make_double3(vj.x, vj.y, vj.z), vj.w, make_double3(abj.x, abj.y, abj.z), tj, rhoj,
+                     gk_t<double>(r2, kh), gk_dr2(r2, kh), acc);
+    }
+  }
+  combine_lanes<LANES>(acc, red);
+  if (!on || sub != 0) return;
+  adj_accel_own(d, b, i, M, o.ti, o.rhoi, irho2i, acc);
+}
+
+// from the tile's LDS copy: 136 bytes per staged particle, one block per CU;
+// the lanes' partial sums reuse the records' space
+__global__ __launch_bounds__(kBlock *kLanesLds64) void k_adj_accel_lds(Dev d, AdjSlot s0, AdjBufs b) {
+  constexpr int NT = kBlock * kLanesLds64;
+  __shared__ double2 r[8 * kStageMax];
+  __shared__ double rh[kStageMax];
+  static_assert(16 * kStageMax >= (kLanesLds64 - 1) * 13 * kBlock, "the partial sums fit the records' space");
+  const int t = xcd_tile(blockIdx.x, gridDim.x), sub = threadIdx.x / kBlock;
+  const int i = t * kBlock + (int)(threadIdx.x % kBlock);
+  const int U = s0.stage_cnt[t];
+  const bool on = i < d.n && d.group[i] >= 0;
+  const int cnt = on ? s0.nnb[i] : 0;
+  const DevMat &M = d.mats[on ? d.mat[i] : 0];
+  const double4 xi = s0.xh[i];
+  AdjAccOwn o{};
+  o.acs = M.alpha * M.Cs, o.beta = M.beta, o.av = M.alpha != 0.0 || M.beta != 0.0;
+  o.vi = s0.vm[i], o.abi = b.ab[i];
+  double irho2i;
+  sigma_t(b, on ? i : 0, o.ti, o.rhoi, irho2i);
+  const GkD k = gk_consts64(xi.w, 3);
+  double acc[13] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  auto pair = [&](const double3 &x, const double3 &u, double m, const double3 &ab, const double (&tj)[6], double rhoj) {
+    const double3 e = make_double3(xi.x - x.x, xi.y - x.y, xi.z - x.z);
+    const double r2 = e.x * e.x + e.y * e.y + e.z * e.z;
+    double GK, dGK;
+    gk_both(r2, k, GK, dGK);
+    adj_accel_pair(o, e, r2, xi.w, u, m, ab, tj, rhoj, GK, dGK, acc);
+  };
+  if (U < 0) {
+    const HbmRows rows{reinterpret_cast<const int4 *>(s0.nbr) + i, d.npad, i};
+    walk_groups<kLanesLds64>(rows, cnt, sub, rows.self(), rows.group(2 * sub), rows.group(2 * sub + 1), [&](const int4 &c) {
+#pragma unroll 1
+      for (int q = 0; q < 4; ++q) {
+        const int j = entry(c, q);
+        const double4 x = s0.xh[j], v = s0.vm[j], ab = b.ab[j];
+        double tj[6], rhoj, irho2j;
+        sigma_t(b, j, tj, rhoj, irho2j);
+        pair(make_double3(x.x, x.y, x.z), make_double3(v.x, v.y, v.z), v.w, make_double3(ab.x, ab.y, ab.z), tj, rhoj);
+      }
+    });
+  } else {
+    const LdsRows rows{reinterpret_cast<const ushort4 *>(s0.nbrl) + i, d.npad, (int)s0.selfl[i]};
+    const ushort4 a0 = rows.group(2 * sub), b0 = rows.group(2 * sub + 1);
+    stage_set<NT>(s0.stage, t, U, [&](int p, int j) {
+      const double4 x = s0.xh[j], v = s0.vm[j], ab = b.ab[j], t0 = b.tsig[2 * j], t1 = b.tsig[2 * j + 1];
+      r[p] = make_double2(x.x, x.y);
+      r[kStageMax + p] = make_double2(x.z, v.w);
+      r[2 * kStageMax + p] = make_double2(v.x, v.y);
+      r[3 * kStageMax + p] = make_double2(v.z, ab.z);
+      r[4 * kStageMax + p] = make_double2(ab.x, ab.y);
+      r[5 * kStageMax + p] = make_double2(t0.x, t0.y);
+      r[6 * kStageMax + p] = make_double2(t0.z, t0.w);
+      r[7 * kStageMax + p] = make_double2(t1.x, t1.y);
+      rh[p] = t1.z;
+    });
+    walk_groups<kLanesLds64>(rows, cnt, sub, rows.self(), a0, b0, [&](const ushort4 &c) {
+#pragma unroll 1
+      for (int q = 0; q < 4; ++q) {
+        const int p = entry(c, q);
+        const double2 x = r[p], z = r[kStageMax + p], u = r[2 * kStageMax + p], w = r[3 * kStageMax + p];
+        const double2 ab = r[4 * kStageMax + p], t0 = r[5 * kStageMax + p], t1 = r[6 * kStageMax + p],
+                      t2 = r[7 * kStageMax + p];
+        const double tj[6] = {t0.x, t0.y, t1.x, t1.y, t2.x, t2.y};
+        pair(make_double3(x.x, x.y, z.x), make_double3(u.x, u.y, w.x), z.y, make_double3(ab.x, ab.y, w.y), tj, rh[p]);
+      }
+    });
+  }
+  __syncthreads();  // the records are read before the partial sums overwrite them
+  combine_lanes<kLanesLds64>(acc, reinterpret_cast<double *>(r));
+  if (on && sub == 0) adj_accel_own(d, b, i, M, o.ti, o.rhoi, irho2i, acc);
+}
+
 void launch_adj_step(const Dev &d, hipStream_t st, const AdjSlot &s0, const AdjSlot &s1, const AdjBufs &b,
                      const BcTable &bc, const AdjSeeds &seeds, double dt, double kick, int adj_mat) {
   const int nb = nblk(d.n);
   constexpr int L = kAdjLanes;
   k_adj_tsig<<<nb, kBlock, 0, st>>>(d, s0, b);
   k_adj_stress<<<nb, kBlock, 0, st>>>(d, s0, b, dt, adj_mat);
-  k_adj_rates<L><<<nb, kBlock * L, 0, st>>>(d, s0, s1, b, dt);
+  if (d.lds64) k_adj_rates_lds<<<nb, kBlock * kLanesLds64, 0, st>>>(d, s0, s1, b, dt);
+  else k_adj_rates<L><<<nb, kBlock * L, 0, st>>>(d, s0, s1, b, dt);
   k_adj_dens<L><<<nb, kBlock * L, 0, st>>>(d, s0, s1, b, bc, seeds, kick);
   if (d.contact) k_adj_contact<<<nb, kBlock, 0, st>>>(d, s0, b, seeds, dt);
-  k_adj_accel<L><<<nb, kBlock * L, 0, st>>>(d, s0, b);
+  if (d.lds64) k_adj_accel_lds<<<nb, kBlock * kLanesLds64, 0, st>>>(d, s0, b);
+  else k_adj_accel<L><<<nb, kBlock * L, 0, st>>>(d, s0, b);
 }
 
 // parameter adjoints: fixed-order block partials, then one block
@@ -651,21 +854,28 @@ void launch_adj_reduce(const Dev &d, hipStream_t st, const AdjBufs &b, double *o
 WF_KERNEL void k_tape_lists(Dev d, AdjSlot s, int force, int *ver, int slot) {
   if (!(force || d.flags->do_search)) return;
   const long long np = d.npad;
-  const long long nrow = (long long)nb_rows(d.max_nb) * np;
   const long long stride = (long long)gridDim.x * kBlock;
   const long long t0 = (long long)blockIdx.x * kBlock + threadIdx.x;
-  for (long long k = t0; k < nrow; k += stride) s.nbr[k] = d.nbr[k];
-  for (long long k = t0; k < np; k += stride) {
-    s.nnb[k] = d.nnb[k];
-    if (d.contact) {
-      s.ccnt[k] = d.ccnt[k];
-      s.id[k] = d.id[k];
-    } else {
-      s.id[k] = d.id[k];
-    }
+  // the rows up to the longest one (npad and the row groups are multiples of
+  // four entries, so every list is a whole number of 16-byte words)
+  const long long ng = (min(d.flags->max_count, d.max_nb) + 3) / 4;
+  auto copy = [&](void *dst, const void *src, long long bytes) {
+    for (long long k = t0; k < bytes / 16; k += stride)
+      reinterpret_cast<int4 *>(dst)[k] = reinterpret_cast<const int4 *>(src)[k];
+  };
+  copy(s.nbr, d.nbr, ng * np * 16);
+  copy(s.nnb, d.nnb, np * 4);
+  copy(s.id, d.id, np * 4);
+  if (d.nbrl) {
+    copy(s.nbrl, d.nbrl, ng * np * 8);
+    copy(s.selfl, d.selfl, np * 2);
+    copy(s.stage, d.stage, (long long)d.ntiles * kStageMax * 4);
   }
-  if (d.contact)
-    for (long long k = t0; k < (long long)kMaxContact * np; k += stride) s.cidx[k] = d.cidx[k];
+  for (long long k = t0; k < d.ntiles; k += stride) s.stage_cnt[k] = d.stage_cnt[k];
+  if (d.contact) {
+    copy(s.ccnt, d.ccnt, np * 4);
+    copy(s.cidx, d.cidx, (long long)kMaxContact * np * 4);
+  }
   if (t0 == 0) ver[slot] = 1;
 }
 void launch_tape_lists(const Dev &d, hipStream_t st, const AdjSlot &s, int force, int *ver, int slot) {

@@ -1188,6 +1188,12 @@ AdjSlot alloc_slot(Ctx *c, bool inter) {
   s.rr = c->adj_alloc<double>(3 * np);
   s.nbr = c->adj_alloc<int>((size_t)nb_rows(c->cfg.max_nb) * np);
   s.nnb = c->adj_alloc<int>(np);
+  if (d.nbrl) {
+    s.nbrl = c->adj_alloc<uint16_t>((size_t)nb_rows(c->cfg.max_nb) * np);
+    s.selfl = c->adj_alloc<uint16_t>(np);
+    s.stage = c->adj_alloc<int>((size_t)d.ntiles * kStageMax);
+  }
+  s.stage_cnt = c->adj_alloc<int>((size_t)d.ntiles);
   s.id = c->adj_alloc<int>(np);
   s.cidx = c->adj_alloc<int>(d.contact ? (size_t)kMaxContact * np : 1);
   s.ccnt = c->adj_alloc<int>(d.contact ? np : 1);
@@ -2421,6 +2427,10 @@ int wf_adj_backward(void *ctx, double *grad) {
         while (v > 0 && !ver[v]) --v;
         s0.nbr = A.slot[v].nbr;
         s0.nnb = A.slot[v].nnb;
+        s0.nbrl = A.slot[v].nbrl;
+        s0.selfl = A.slot[v].selfl;
+        s0.stage = A.slot[v].stage;
+        s0.stage_cnt = A.slot[v].stage_cnt;
         s0.id = A.slot[v].id;
         s0.cidx = A.slot[v].cidx;
         s0.ccnt = A.slot[v].ccnt;

@@ -199,6 +199,112 @@ __device__ inline R gk_t(R r2, const KH<R> &k) {
 }
 
 
+// the FP64 row walks' gradient factor: its constants, and reciprocals
+struct GkD {
+  double ih, gin_a, gin_b, gout;  // 1/h, 2.25 c5, -3 c5, -0.75 c5 h
+};
+__device__ inline GkD gk_consts64(double h, int dim) {
+  const KH<double> k = kern_h_t<double>(h, dim);
+  return GkD{k.ih, 2.25 * k.c5, -3.0 * k.c5, -0.75 * k.c5 * h};
+}
+// 1/x and 1/sqrt(x): the hardware estimate (relative error d < 2^-23) and one
+// third-order step, 1/x = y / (1 - e) = y (1 + e + e^2 + ...) with
+// e = 1 - x y, and the series of (1 - e)^(-1/2): errors d^3 and below, under
+// the rounding
+__device__ inline double rcp3(double x) {
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(y, fma(e, e, e), y);
+}
+__device__ inline double rsqrt3(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+// ---------------------------------------------------------------------------
+// neighbour rows read in groups of four entries, and a tile's staged set
+
+struct LdsRows {
+  using G = ushort4;
+  const ushort4 *row;
+  long long np;
+  int own;  // the particle's position in the staged set
+  __device__ G group(int g) const { return row[(long long)g * np]; }
+  __device__ G self() const {
+    const unsigned short o = (unsigned short)own;
+    return make_ushort4(o, o, o, o);
+  }
+};
+struct HbmRows {
+  using G = int4;
+  const int4 *row;
+  long long np;
+  int own;  // the particle's index
+  __device__ G group(int g) const { return row[(long long)g * np]; }
+  __device__ G self() const { return make_int4(own, own, own, own); }
+};
+template <class G>
+__device__ inline int entry(const G &c, int u) {
+  return u == 0 ? (int)c.x : (u == 1 ? (int)c.y : (u == 2 ? (int)c.z : (int)c.w));
+}
+
+// Lane `sub` of LANES takes the group pairs (2k, 2k + 1) with k = sub,
+// sub + LANES, ...: a row of ng groups costs its lanes ng groups in all
+// (the second group of the last pair is a self group when ng is odd).  An
+// iteration processes one pair, the next pair's row words loaded at its top
+// so they are in flight while this pair is processed.  The iteration is one
+// branch-free block (a branch between the groups lets the compiler sink the
+// prefetch down to its use): a second group past the row's end is replaced
+// by `self`, a group of four self entries, whose pair terms are zeros.  The
+// groups beyond a row's end that the prefetch touches (at most 2 LANES + 1)
+// lie inside the allocation (nb_rows keeps kRowSpare spare entries) and are
+// never used.
+// a, b: the lane's first two groups (rows.group(2 sub) and the next), which
+// the kernels load before they stage the tile.
+template <int LANES, class Rows, class F>
+__device__ inline void walk_groups(const Rows &rows, int cnt, int sub, const typename Rows::G &self,
+                                   typename Rows::G a, typename Rows::G b, F &&group_fn) {
+  static_assert(4 * (2 * LANES + 2) <= kRowSpare, "prefetch stays in the row allocation");
+  const int ng = (cnt + 3) >> 2;
+  for (int g = 2 * sub; g < ng; g += 2 * LANES) {
+    const typename Rows::G a2 = rows.group(g + 2 * LANES);
+    const typename Rows::G b2 = rows.group(g + 2 * LANES + 1);
+    // compiler-only barrier: the prefetch stays issued here (it may not be
+    // re-formed as a load next to its use); emits no instruction
+    asm volatile("" ::: "memory");
+    group_fn(a);
+    // the second group's loads are not hoisted over the first group's
+    // arithmetic (that would hold both groups' records in registers)
+    __builtin_amdgcn_sched_barrier(0);
+    group_fn(g + 1 < ng ? b : self);
+    // the register moves of the hand-over stay at the end of the iteration
+    // (moved earlier they would wait for the prefetch)
+    __builtin_amdgcn_sched_barrier(0);
+    a = a2;
+    b = b2;
+  }
+}
+
+
+// all NT threads call put(p, j) for the entries of tile t's staged set (each
+// thread's indices are loaded first), then meet at a barrier
+template <int NT, class F>
+__device__ inline void stage_set(const int *stage, int t, int U, F &&put) {
+  constexpr int R = (kStageMax + NT - 1) / NT;
+  const int *st = stage + (long long)t * kStageMax;
+  int j[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int p = (int)threadIdx.x + q * NT;
+    j[q] = p < U ? st[p] : -1;
+  }
+#pragma unroll
+  for (int q = 0; q < R; ++q)
+    if (j[q] >= 0) put((int)threadIdx.x + q * NT, j[q]);
+  __syncthreads();
+}
+
 // amplitude::getValAtTime (Source/Domain.h:75-87)
 __device__ inline double amp_value(const DevAmp &a, double t) {
   int i = a.n - 1;

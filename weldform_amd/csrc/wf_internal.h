@@ -338,6 +338,8 @@ struct AdjSlot {
   double4 *apre;               // acceleration after the pair pass (before contact)
   double *drho, *sr, *rr;      // density rate, strain rate [6], rotation rate [3]
   int *nbr, *nnb;              // neighbour list in effect
+  uint16_t *nbrl, *selfl;      // and its staging lists, where the passes read from LDS
+  int *stage, *stage_cnt;
   int *cidx, *ccnt, *id;       // contact partners and particle ids in effect
   double4 *node, *enorm, *rv;  // rigid planes at the step's contact evaluation
 };
