@@ -12,7 +12,6 @@
 #include <cstring>
 #include <stdexcept>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -1609,7 +1608,8 @@ static void copy_out(Ctx *c, void *dst, const void *src, size_t bytes) {
   std::atomic<size_t> next{0};
   std::atomic<int> err{(int)hipSuccess};
   auto work = [&](int t) {
-    hipError_t e = hipSetDevice(c->cfg.device);
+    // (the caller's own thread keeps its current device)
+    hipError_t e = t > 0 ? hipSetDevice(c->cfg.device) : hipSuccess;
     for (size_t k = next++; e == hipSuccess && k < nch; k = next++) {
       const size_t off = k * kCopyChunk, len = std::min(kCopyChunk, bytes - off);
       e = hipMemcpyAsync(c->pin[t], (const char *)src + off, len, hipMemcpyDeviceToHost, c->st);
@@ -1623,7 +1623,7 @@ static void copy_out(Ctx *c, void *dst, const void *src, size_t bytes) {
   team.reserve(nt);
   try {
     for (int t = 1; t < nt; ++t) team.emplace_back(work, t);
-  } catch (const std::system_error &) {
+  } catch (...) {
     // fewer threads: the others take the chunks
   }
   work(0);
