@@ -820,7 +820,7 @@ WF_KERNEL void k_build_nbr_wide(Dev d, int cur) {
   }
 }
 
-// LDS staging lists of the mixed-precision pair passes, per tile of kBlock
+// LDS staging lists of the pair passes, per tile of kBlock
 // consecutive particles after every neighbour build: the tile's particles
 // and all their neighbour entries go into an LDS hash set (open
 // addressing); its distinct values (the staged set, ~6 % of the ~7000
