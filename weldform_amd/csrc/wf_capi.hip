@@ -1085,10 +1085,12 @@ void enqueue_step(Ctx *c, int scheme, int cur, const TapeHook *tp = nullptr, int
       }
       if (d.contact && split) launch_rigid_drift(d, c->st, dt);
     }
+    bool stress;
     {
       Timed t(c, T_RATES);
-      launch_rates(d, c->st, nxt, dt, 1);
+      stress = launch_rates(d, c->st, nxt, dt, 1);
     }
+    if (!stress) launch_stress(d, c->st, nxt, dt);
     if (c->cfg.thermal_solver) launch_thermal(d, c->st, nxt);
     launch_finalize(d, c->st, dt, c->bc.nz, split ? 0 : 1);
     if (tp) {

@@ -385,8 +385,9 @@ void launch_kick(const Dev &d, hipStream_t st, const BcTable &bc, int scheme, do
 void launch_time_step(const Dev &d, hipStream_t st, int cur);
 void launch_kick2(const Dev &d, hipStream_t st, double dt);
 void launch_dens_drift(const Dev &d, hipStream_t st, int cur, double dt, int do_update);
-// do_stress: with the stress update of every particle (a step of size dt)
-void launch_rates(const Dev &d, hipStream_t st, int buf, double dt, int do_stress);
+// do_stress: with the stress update of every particle (a step of size dt) where
+// the rate kernel takes it; returns whether it did (else launch_stress follows)
+bool launch_rates(const Dev &d, hipStream_t st, int buf, double dt, int do_stress);
 void launch_stress(const Dev &d, hipStream_t st, int buf, double dt);
 void launch_thermal(const Dev &d, hipStream_t st, int buf);
 // the end-of-step sums and the rigid meshes' update; drift: with the rigid

@@ -2881,12 +2881,8 @@ WF_KERNEL void k_stress(Dev d, int buf, double dt) {
 // particles 11.3 and 15.5 us, 35k 16.2 and 22.7; 56k (FP64) 26.6 and 32, but a
 // damage step 2 % slower; 370k 84 and 85, 954k 200 and 194 (FP64 301 and 272).
 constexpr int kFuseTiles = 320;
-void launch_rates(const Dev &d, hipStream_t st, int buf, double dt, int do_stress) {
-  if (do_stress && d.ntiles > kFuseTiles) {
-    launch_rates(d, st, buf, dt, 0);
-    launch_stress(d, st, buf, dt);
-    return;
-  }
+bool launch_rates(const Dev &d, hipStream_t st, int buf, double dt, int do_stress) {
+  if (d.ntiles > kFuseTiles) do_stress = 0;
   if (d.mixed) {
     WF_LANES_GC_SWITCH(d.lanes_mx, d.gc_on, k_rates_mx, d, buf, dt, do_stress)
   } else {
@@ -2898,6 +2894,7 @@ void launch_rates(const Dev &d, hipStream_t st, int buf, double dt, int do_stres
       WF_LANES_SWITCH(d.lanes_f64, k_rates_f64, d, buf, dt, do_stress)
     }
   }
+  return do_stress != 0;
 }
 
 void launch_stress(const Dev &d, hipStream_t st, int buf, double dt) {
