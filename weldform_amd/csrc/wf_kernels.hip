@@ -2855,7 +2855,7 @@ __global__ __launch_bounds__(kBlock *LANES) void k_rates_mx(Dev d, int buf, doub
   rates_finish<true, LANES>(d, i, sub, v, own, dt, do_stress, reinterpret_cast<float *>(lx), sh);
 }
 
-// the stress update alone (single-pass evaluations)
+// the stress update alone (single-pass evaluations; the step above kFuseTiles tiles)
 template <bool MX>
 WF_KERNEL void k_stress(Dev d, int buf, double dt) {
   __shared__ double sh[5 * kBlock / 64];
