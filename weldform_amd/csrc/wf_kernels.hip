@@ -2858,6 +2858,7 @@ __global__ __launch_bounds__(kBlock *LANES) void k_rates_mx(Dev d, int buf, doub
 // the stress update alone (single-pass evaluations; the step above kFuseTiles tiles)
 template <bool MX>
 WF_KERNEL void k_stress(Dev d, int buf, double dt) {
+  if (dt < 0) dt = d.flags->dt;
   __shared__ double sh[5 * kBlock / 64];
   const int i = blockIdx.x * kBlock + threadIdx.x;
   const long long np = d.npad;
