@@ -326,7 +326,7 @@ __global__ __launch_bounds__(kBlock *kLanesLds64) void k_adj_rates_lds(Dev d, Ad
   __shared__ double red[(kLanesLds64 - 1) * 7 * kBlock];
   const int t = xcd_tile(blockIdx.x, gridDim.x), sub = threadIdx.x / kBlock;
   const int i = t * kBlock + (int)(threadIdx.x % kBlock);
-  const int U = s0.stage_cnt[t];
+  const int U = d.stage_cnt[t];
   const bool on = i < d.n;
   const int cnt = on && d.group[i] >= 0 ? s0.nnb[i] : 0;
   const double4 xi = s1.xh[i], vi = s1.vm[i];
@@ -355,9 +355,9 @@ __global__ __launch_bounds__(kBlock *kLanesLds64) void k_adj_rates_lds(Dev d, Ad
       }
     });
   } else {
-    const LdsRows rows{reinterpret_cast<const ushort4 *>(s0.nbrl) + i, d.npad, (int)s0.selfl[i]};
+    const LdsRows rows{reinterpret_cast<const ushort4 *>(d.nbrl) + i, d.npad, (int)d.selfl[i]};
     const ushort4 a0 = rows.group(2 * sub), b0 = rows.group(2 * sub + 1);
-    stage_set<NT>(s0.stage, t, U, [&](int p, int j) {
+    stage_set<NT>(d.stage, t, U, [&](int p, int j) {
       const double4 x = s1.xh[j], v = s1.vm[j], a = b.rsb[3 * j], c = b.rsb[3 * j + 1];
       const double w12 = b.rsb[3 * j + 2].x;
       r[p] = make_double2(x.x, x.y);
@@ -747,7 +747,7 @@ __global__ __launch_bounds__(kBlock *kLanesLds64) void k_adj_accel_lds(Dev d, Ad
   static_assert(16 * kStageMax >= (kLanesLds64 - 1) * 13 * kBlock, "the partial sums fit the records' space");
   const int t = xcd_tile(blockIdx.x, gridDim.x), sub = threadIdx.x / kBlock;
   const int i = t * kBlock + (int)(threadIdx.x % kBlock);
-  const int U = s0.stage_cnt[t];
+  const int U = d.stage_cnt[t];
   const bool on = i < d.n && d.group[i] >= 0;
   const int cnt = on ? s0.nnb[i] : 0;
   const DevMat &M = d.mats[on ? d.mat[i] : 0];
@@ -779,9 +779,9 @@ __global__ __launch_bounds__(kBlock *kLanesLds64) void k_adj_accel_lds(Dev d, Ad
       }
     });
   } else {
-    const LdsRows rows{reinterpret_cast<const ushort4 *>(s0.nbrl) + i, d.npad, (int)s0.selfl[i]};
+    const LdsRows rows{reinterpret_cast<const ushort4 *>(d.nbrl) + i, d.npad, (int)d.selfl[i]};
     const ushort4 a0 = rows.group(2 * sub), b0 = rows.group(2 * sub + 1);
-    stage_set<NT>(s0.stage, t, U, [&](int p, int j) {
+    stage_set<NT>(d.stage, t, U, [&](int p, int j) {
       const double4 x = s0.xh[j], v = s0.vm[j], ab = b.ab[j], t0 = b.tsig[2 * j], t1 = b.tsig[2 * j + 1];
       r[p] = make_double2(x.x, x.y);
       r[kStageMax + p] = make_double2(x.z, v.w);
@@ -866,12 +866,6 @@ WF_KERNEL void k_tape_lists(Dev d, AdjSlot s, int force, int *ver, int slot) {
   copy(s.nbr, d.nbr, ng * np * 16);
   copy(s.nnb, d.nnb, np * 4);
   copy(s.id, d.id, np * 4);
-  if (d.nbrl) {
-    copy(s.nbrl, d.nbrl, ng * np * 8);
-    copy(s.selfl, d.selfl, np * 2);
-    copy(s.stage, d.stage, (long long)d.ntiles * kStageMax * 4);
-  }
-  for (long long k = t0; k < d.ntiles; k += stride) s.stage_cnt[k] = d.stage_cnt[k];
   if (d.contact) {
     copy(s.ccnt, d.ccnt, np * 4);
     copy(s.cidx, d.cidx, (long long)kMaxContact * np * 4);

@@ -101,6 +101,9 @@ struct Ctx {
   long long gsum_cap = 0;
   Dev d{};
   std::vector<std::pair<void *, size_t>> allocs;  // (pointer, bytes) of the solver state
+  // the staging lists (k_stage's: stage_cnt, stage, nbrl, selfl): a function of
+  // the neighbour rows, so no part of the adjoint's snapshots and tape
+  std::vector<void *> lists;
   DevMat *dmats = nullptr;
   int cur = 0;
   double dt = 0.0;  // the initial step (Domain::deltatint); the device flags hold the current one
@@ -131,6 +134,14 @@ struct Ctx {
     HIPCHK(hipMalloc(&p, count * sizeof(T)));
     HIPCHK(hipMemsetAsync(p, 0, count * sizeof(T), st));
     allocs.push_back({p, count * sizeof(T)});
+    return (T *)p;
+  }
+  template <class T>
+  T *list_alloc(size_t count) {
+    void *p = nullptr;
+    HIPCHK(hipMalloc(&p, count * sizeof(T)));
+    lists.push_back(p);
+    HIPCHK(hipMemsetAsync(p, 0, count * sizeof(T), st));
     return (T *)p;
   }
   // adjoint storage: checkpoints, tape, adjoint buffers (not part of the
@@ -180,6 +191,7 @@ struct Ctx {
     drop_graphs();
     for (auto &e : ev_pool) (void)hipEventDestroy(e);
     for (auto &p : allocs) (void)hipFree(p.first);
+    for (void *p : lists) (void)hipFree(p);
     for (void *p : adj.mem) (void)hipFree(p);
     if (outbuf) (void)hipFree(outbuf);
     for (void *p : pin) (void)hipHostFree(p);
@@ -622,14 +634,14 @@ void allocate(Ctx *c) {
     dput(c, d.gcm, eye);
   }
   // stage_cnt = -1 marks a tile that gathers from HBM
-  d.stage_cnt = c->alloc<int>((size_t)d.ntiles);
+  d.stage_cnt = c->list_alloc<int>((size_t)d.ntiles);
   HIPCHK(hipMemsetAsync(d.stage_cnt, 0xff, sizeof(int) * (size_t)d.ntiles, c->st));
   choose_f64(c);
   if (c->cfg.stage_max >= 0 && (d.mixed || d.lds64)) {
     d.stage_max = c->cfg.stage_max == 0 ? kStageMax : c->cfg.stage_max;
-    d.stage = c->alloc<int>((size_t)d.ntiles * kStageMax);
-    d.nbrl = c->alloc<uint16_t>((size_t)nb_rows(c->cfg.max_nb) * np);
-    d.selfl = c->alloc<uint16_t>(np);
+    d.stage = c->list_alloc<int>((size_t)d.ntiles * kStageMax);
+    d.nbrl = c->list_alloc<uint16_t>((size_t)nb_rows(c->cfg.max_nb) * np);
+    d.selfl = c->list_alloc<uint16_t>(np);
   }
   // per-group sums: each material index's particles in internal order
   d.ngroups = 0;
@@ -1170,6 +1182,7 @@ void restore(Ctx *c, size_t k) {
   }
   c->cur = c->adj.ckh[k].first;
   c->steps = c->adj.ckh[k].second;
+  launch_stage(c->d, c->st);
 }
 
 AdjSlot alloc_slot(Ctx *c, bool inter) {
@@ -1189,12 +1202,6 @@ AdjSlot alloc_slot(Ctx *c, bool inter) {
   s.rr = c->adj_alloc<double>(3 * np);
   s.nbr = c->adj_alloc<int>((size_t)nb_rows(c->cfg.max_nb) * np);
   s.nnb = c->adj_alloc<int>(np);
-  if (d.nbrl) {
-    s.nbrl = c->adj_alloc<uint16_t>((size_t)nb_rows(c->cfg.max_nb) * np);
-    s.selfl = c->adj_alloc<uint16_t>(np);
-    s.stage = c->adj_alloc<int>((size_t)d.ntiles * kStageMax);
-  }
-  s.stage_cnt = c->adj_alloc<int>((size_t)d.ntiles);
   s.id = c->adj_alloc<int>(np);
   s.cidx = c->adj_alloc<int>(d.contact ? (size_t)kMaxContact * np : 1);
   s.ccnt = c->adj_alloc<int>(d.contact ? np : 1);
@@ -2422,17 +2429,22 @@ int wf_adj_backward(void *ctx, double *grad) {
       }
       tape_state(c, A.slot[len], c->cur);
       const auto ver = dget(c, A.ver, (size_t)len);
-      // reverse sweep over the segment
+      // reverse sweep over the segment; the staging lists follow the rows of
+      // the step in hand (at first the replay's last)
+      int staged = -1;
       for (int s = len - 1; s >= 0; --s) {
         AdjSlot s0 = A.slot[s];
         int v = s;
         while (v > 0 && !ver[v]) --v;
+        if (staged >= 0 && v != staged) {
+          Dev rows = d;
+          rows.nbr = A.slot[v].nbr;
+          rows.nnb = A.slot[v].nnb;
+          launch_stage(rows, c->st);
+        }
+        staged = v;
         s0.nbr = A.slot[v].nbr;
         s0.nnb = A.slot[v].nnb;
-        s0.nbrl = A.slot[v].nbrl;
-        s0.selfl = A.slot[v].selfl;
-        s0.stage = A.slot[v].stage;
-        s0.stage_cnt = A.slot[v].stage_cnt;
         s0.id = A.slot[v].id;
         s0.cidx = A.slot[v].cidx;
         s0.ccnt = A.slot[v].ccnt;

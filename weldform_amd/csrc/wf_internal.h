@@ -338,8 +338,6 @@ struct AdjSlot {
   double4 *apre;               // acceleration after the pair pass (before contact)
   double *drho, *sr, *rr;      // density rate, strain rate [6], rotation rate [3]
   int *nbr, *nnb;              // neighbour list in effect
-  uint16_t *nbrl, *selfl;      // and its staging lists, where the passes read from LDS
-  int *stage, *stage_cnt;
   int *cidx, *ccnt, *id;       // contact partners and particle ids in effect
   double4 *node, *enorm, *rv;  // rigid planes at the step's contact evaluation
 };
@@ -369,6 +367,8 @@ void launch_tape_lists(const Dev &d, hipStream_t st, const AdjSlot &s, int force
 void launch_schedule(const Dev &d, hipStream_t st, int force, const BcTable *bc);
 void launch_plane_strain(const Dev &d, hipStream_t st);
 void launch_neighbours(const Dev &d, hipStream_t st, int cur);
+// the staging lists of the rows d.nbr, d.nnb as they are, without a search
+void launch_stage(const Dev &d, hipStream_t st);
 void launch_gradcorr(const Dev &d, hipStream_t st, int cur);
 void launch_accel(const Dev &d, hipStream_t st, int cur);
 void launch_tir(const Dev &d, hipStream_t st, int cur);

@@ -889,8 +889,8 @@ __device__ inline void stage_sort(int (&v)[4], int P, int *buf) {
   }
 }
 
-__global__ __launch_bounds__(kStageThreads) void k_stage(Dev d) {
-  if (!d.flags->do_search) return;
+__global__ __launch_bounds__(kStageThreads) void k_stage(Dev d, int force) {
+  if (!force && !d.flags->do_search) return;
   __shared__ int uniq[kStagePow2];
   __shared__ int ht[kHashSlots];
   __shared__ unsigned short hp[kHashSlots];
@@ -1104,7 +1104,10 @@ void launch_neighbours(const Dev &d, hipStream_t st, int cur) {
   }
   if (d.n <= kBuildWide) k_build_nbr_wide<<<nblk((long long)d.n * kBuildLanes), kBlock, 0, st>>>(d, cur);
   else k_build_nbr<<<nblk(d.n), kBlock, 0, st>>>(d, cur);
-  if (d.stage_max > 0) k_stage<<<d.ntiles < 2048 ? d.ntiles : 2048, kStageThreads, 0, st>>>(d);
+  if (d.stage_max > 0) k_stage<<<d.ntiles < 2048 ? d.ntiles : 2048, kStageThreads, 0, st>>>(d, 0);
+}
+void launch_stage(const Dev &d, hipStream_t st) {
+  if (d.stage_max > 0) k_stage<<<d.ntiles < 2048 ? d.ntiles : 2048, kStageThreads, 0, st>>>(d, 1);
 }
 
 // ---------------------------------------------------------------------------
