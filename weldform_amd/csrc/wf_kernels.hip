@@ -1113,8 +1113,10 @@ void launch_stage(const Dev &d, hipStream_t st) {
 // ---------------------------------------------------------------------------
 // pass 1: acceleration (CalcAccel + AccelReduction, GradientType 0, TI = 0)
 
-// P / rho^2 with the equation of state's P
+// P / rho^2 with the equation of state's P.  Rounded here, not fused into the
+// sum that takes it: a neighbour's value is the same from HBM and from LDS
 __device__ inline double pr_of(double rho, double P0, double cs2, double rho0) {
+#pragma clang fp contract(off)
   const double ir = rcp_t(rho);
   return (P0 + cs2 * (rho - rho0)) * ir * ir;
 }
