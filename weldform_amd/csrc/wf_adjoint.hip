@@ -46,7 +46,11 @@ __device__ inline double gk_dr2(double r2, const KH<double> &k) {
 
 // GK and d GK / d r2 together, without branches (r2 = 0, a padding entry of the
 // particle itself: every pair term it enters is an exact zero)
+// (this and the pair terms below fuse within an expression only: the copies
+// compiled for records from LDS and from HBM then round alike, and the gradient
+// does not depend on which tiles are staged)
 __device__ inline void gk_both(double r2, const GkD &k, double &GK, double &dGK) {
+#pragma clang fp contract(on)
   const double ri = rsqrt3(fmax(r2, DBL_MIN));
   const double q = (r2 * ri) * k.ih;
   const double t = fmax(2.0 - q, 0.0);
@@ -226,6 +230,7 @@ __device__ inline void rate_seeds(const AdjBufs &b, int j, double sb[6], double 
 __device__ inline void adj_rates_pair(const double3 &e3, const double4 &vi, const double3 &uj, double voli, double volj,
                                       const double (&sbi)[6], const double (&wbi)[3], const double (&sbj)[6],
                                       const double (&wbj)[3], double GK, double dGK, double (&acc)[7]) {
+#pragma clang fp contract(on)
   const double dx = e3.x, dy = e3.y, dz = e3.z;
   const double vx = vi.x - uj.x, vy = vi.y - uj.y, vz = vi.z - uj.z;
   const double cp = -0.5 * GK;
@@ -337,6 +342,7 @@ __global__ __launch_bounds__(kBlock *kLanesLds64) void k_adj_rates_lds(Dev d, Ad
   const GkD k = gk_consts64(xi.w, 3);
   double acc[7] = {0, 0, 0, 0, 0, 0, 0};
   auto pair = [&](const double3 &x, const double3 &u, double vol, const double (&sbj)[6], const double (&wbj)[3]) {
+#pragma clang fp contract(on)
     const double3 e = make_double3(xi.x - x.x, xi.y - x.y, xi.z - x.z);
     double GK, dGK;
     gk_both(e.x * e.x + e.y * e.y + e.z * e.z, k, GK, dGK);
@@ -639,6 +645,7 @@ struct AdjAccOwn {
 __device__ inline void adj_accel_pair(const AdjAccOwn &o, const double3 &e3, double r2, double h, const double3 &uj,
                                       double mj, const double3 &abj, const double (&tj)[6], double rhoj, double GK,
                                       double dGK, double (&acc)[13]) {
+#pragma clang fp contract(on)
   const double dx = e3.x, dy = e3.y, dz = e3.z;
   const double4 &vi = o.vi, &abi = o.abi;
   const double (&ti)[6] = o.ti;
@@ -760,6 +767,7 @@ __global__ __launch_bounds__(kBlock *kLanesLds64) void k_adj_accel_lds(Dev d, Ad
   const GkD k = gk_consts64(xi.w, 3);
   double acc[13] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   auto pair = [&](const double3 &x, const double3 &u, double m, const double3 &ab, const double (&tj)[6], double rhoj) {
+#pragma clang fp contract(on)
     const double3 e = make_double3(xi.x - x.x, xi.y - x.y, xi.z - x.z);
     const double r2 = e.x * e.x + e.y * e.y + e.z * e.z;
     double GK, dGK;
