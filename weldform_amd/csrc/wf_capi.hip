@@ -101,9 +101,6 @@ struct Ctx {
   long long gsum_cap = 0;
   Dev d{};
   std::vector<std::pair<void *, size_t>> allocs;  // (pointer, bytes) of the solver state
-  // the staging lists (k_stage's: stage_cnt, stage, nbrl, selfl): a function of
-  // the neighbour rows, so no part of the adjoint's snapshots and tape
-  std::vector<void *> lists;
   DevMat *dmats = nullptr;
   int cur = 0;
   double dt = 0.0;  // the initial step (Domain::deltatint); the device flags hold the current one
@@ -136,13 +133,34 @@ struct Ctx {
     allocs.push_back({p, count * sizeof(T)});
     return (T *)p;
   }
+  // The staging lists (k_stage's: d.stage, d.nbrl, d.selfl, and d.stage_cnt):
+  // a function of the neighbour rows, so no part of the adjoint's snapshots and
+  // tape.  FP64 contexts do without them where the device's memory is short:
+  // their passes then read the same records from HBM, with the same results.
   template <class T>
-  T *list_alloc(size_t count) {
-    void *p = nullptr;
-    HIPCHK(hipMalloc(&p, count * sizeof(T)));
-    lists.push_back(p);
+  void list_alloc(T *&p, size_t count) {
+    if (p) (void)hipFree(p);  // (an earlier wf_init that failed)
+    p = nullptr;
+    HIPCHK(hipMalloc((void **)&p, count * sizeof(T)));
     HIPCHK(hipMemsetAsync(p, 0, count * sizeof(T), st));
-    return (T *)p;
+  }
+  void free_lists() {
+    for (void *p : {(void *)d.stage, (void *)d.nbrl, (void *)d.selfl})
+      if (p) (void)hipFree(p);
+    d.stage = nullptr;
+    d.nbrl = d.selfl = nullptr;
+    d.stage_max = 0;
+  }
+  // memory taken after wf_init
+  hipError_t later_malloc(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory || d.mixed || !d.nbrl) return e;
+    (void)hipGetLastError();
+    if ((e = hipStreamSynchronize(st)) != hipSuccess) return e;
+    free_lists();
+    drop_graphs();  // (the captured steps hold the lists)
+    if ((e = hipMemsetAsync(d.stage_cnt, 0xff, sizeof(int) * (size_t)d.ntiles, st)) != hipSuccess) return e;
+    return hipMalloc(p, bytes);
   }
   // adjoint storage: checkpoints, tape, adjoint buffers (not part of the
   // snapshots)
@@ -174,7 +192,7 @@ struct Ctx {
   T *adj_alloc(size_t count) {
     void *p = nullptr;
     if (count == 0) count = 1;
-    HIPCHK(hipMalloc(&p, count * sizeof(T)));
+    HIPCHK(later_malloc(&p, count * sizeof(T)));
     HIPCHK(hipMemsetAsync(p, 0, count * sizeof(T), st));
     adj.mem.push_back(p);
     return (T *)p;
@@ -191,7 +209,8 @@ struct Ctx {
     drop_graphs();
     for (auto &e : ev_pool) (void)hipEventDestroy(e);
     for (auto &p : allocs) (void)hipFree(p.first);
-    for (void *p : lists) (void)hipFree(p);
+    free_lists();
+    if (d.stage_cnt) (void)hipFree(d.stage_cnt);
     for (void *p : adj.mem) (void)hipFree(p);
     if (outbuf) (void)hipFree(outbuf);
     for (void *p : pin) (void)hipHostFree(p);
@@ -634,15 +653,9 @@ void allocate(Ctx *c) {
     dput(c, d.gcm, eye);
   }
   // stage_cnt = -1 marks a tile that gathers from HBM
-  d.stage_cnt = c->list_alloc<int>((size_t)d.ntiles);
+  c->list_alloc(d.stage_cnt, (size_t)d.ntiles);
   HIPCHK(hipMemsetAsync(d.stage_cnt, 0xff, sizeof(int) * (size_t)d.ntiles, c->st));
   choose_f64(c);
-  if (c->cfg.stage_max >= 0 && (d.mixed || d.lds64)) {
-    d.stage_max = c->cfg.stage_max == 0 ? kStageMax : c->cfg.stage_max;
-    d.stage = c->list_alloc<int>((size_t)d.ntiles * kStageMax);
-    d.nbrl = c->list_alloc<uint16_t>((size_t)nb_rows(c->cfg.max_nb) * np);
-    d.selfl = c->list_alloc<uint16_t>(np);
-  }
   // per-group sums: each material index's particles in internal order
   d.ngroups = 0;
   if (c->gsum_zone != -2) {
@@ -679,6 +692,19 @@ void allocate(Ctx *c) {
     if (d.contact) {
       d.gcf = c->alloc<double4>((size_t)kMaxMesh * np);
       d.gc_hist = c->alloc<double>((size_t)d.ghist_cap * ng * kMaxMesh * 3);
+    }
+  }
+  // the staging lists last: what FP64 can do without
+  if (c->cfg.stage_max >= 0 && (d.mixed || d.lds64)) {
+    try {
+      c->list_alloc(d.stage, (size_t)d.ntiles * kStageMax);
+      c->list_alloc(d.nbrl, (size_t)nb_rows(c->cfg.max_nb) * np);
+      c->list_alloc(d.selfl, np);
+      d.stage_max = c->cfg.stage_max == 0 ? kStageMax : c->cfg.stage_max;
+    } catch (const Error &) {
+      if (d.mixed) throw;
+      (void)hipGetLastError();
+      c->free_lists();
     }
   }
 }
@@ -1579,7 +1605,7 @@ static void *out_staging(Ctx *c, size_t bytes) {
       c->outbuf = nullptr;
       c->out_cap = 0;
     }
-    HIPCHK(hipMalloc(&c->outbuf, bytes));
+    HIPCHK(c->later_malloc(&c->outbuf, bytes));
     c->out_cap = bytes;
   }
   return c->outbuf;
