@@ -3076,7 +3076,8 @@ __global__ __launch_bounds__(kBlock *kLanesHeat) void k_thermal_lds(Dev d, int b
   combine_lanes<kLanesHeat>(s, red);
   __builtin_amdgcn_sched_barrier(0);
   double3 e = make_double3(0.0, 0.0, 0.0);
-  if (on && sub == 0) e = thermal_own(d, buf, i, pair_kk(d.mats[d.mat[i]]) * s[0]);
+  // (no pairs, no factor: a conductivity of 0 makes it 0/0)
+  if (on && sub == 0) e = thermal_own(d, buf, i, cnt > 0 ? pair_kk(d.mats[d.mat[i]]) * s[0] : 0.0);
   thermal_sums(d, e, t, sh);
 }
 
