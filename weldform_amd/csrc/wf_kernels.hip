@@ -3950,11 +3950,21 @@ WF_KERNEL void k_rigid_drift(Dev d, double dt) {
   d.rx[r] = x;
 }
 
-constexpr int kSurfSmall = 32768;
+// Blocks of 16 particles spread the partner search of small models over the
+// chip, but cost 2 us on steps without a search once there are a thousand of
+// them.  They are taken up to 32768 particles where the rigid surface is fine
+// against the model (a rigid particle or more for 16 of the model's), so that
+// its particles have many candidates.  Us per step with a search every 5, blocks
+// of 16 against 128 particles, rigid surfaces of 256, 576, 1024, 2304 and, at
+// 18k and 30k, 8192 particles:
+//   1.3k  14 15   19 20   25 28   43 51
+//   9k    14.3 13.9   14.6 15.2   16 17   21 21
+//   18k   15.2 13.7   15.8 15.1   15.5 16.2   19.5 20.6   19 75
+//   30k   16.1 13.7   16.7 14.6   16.7 15.2   18.3 18.7   48 65
+constexpr int kSurfSmall = 32768, kSurfFine = 16;
 void launch_surface(const Dev &d, hipStream_t st, int cur, int setup) {
-  // small models: more, smaller blocks, so that the partner search fills the
-  // chip
-  if (setup == 0 && d.n <= kSurfSmall) k_surface<16><<<(d.n + 15) / 16, kBlock, 0, st>>>(d, cur, setup);
+  if (setup == 0 && d.n <= kSurfSmall && d.n <= kSurfFine * (long long)d.nrig)
+    k_surface<16><<<(d.n + 15) / 16, kBlock, 0, st>>>(d, cur, setup);
   else k_surface<kBlock><<<nblk(d.n), kBlock, 0, st>>>(d, cur, setup);
 }
 void launch_rigid_bc(const Dev &d, hipStream_t st, const BcTable &bc) {
