@@ -145,8 +145,7 @@ struct Ctx {
     HIPCHK(hipMemsetAsync(p, 0, count * sizeof(T), st));
   }
   void free_lists() {
-    for (void *p : {(void *)d.stage, (void *)d.nbrl, (void *)d.selfl})
-      if (p) (void)hipFree(p);
+    if (d.stage) (void)hipFree(d.stage);  // (one allocation holds them)
     d.stage = nullptr;
     d.nbrl = d.selfl = nullptr;
     d.stage_max = 0;
@@ -697,9 +696,11 @@ void allocate(Ctx *c) {
   // the staging lists last: what FP64 can do without
   if (c->cfg.stage_max >= 0 && (d.mixed || d.lds64)) {
     try {
-      c->list_alloc(d.stage, (size_t)d.ntiles * kStageMax);
-      c->list_alloc(d.nbrl, (size_t)nb_rows(c->cfg.max_nb) * np);
-      c->list_alloc(d.selfl, np);
+      // (np is a multiple of kBlock: every part starts 256-byte aligned)
+      const size_t ns = (size_t)d.ntiles * kStageMax, nl = (size_t)nb_rows(c->cfg.max_nb) * np;
+      c->list_alloc(d.stage, ns + (nl + np) / 2);
+      d.nbrl = reinterpret_cast<uint16_t *>(d.stage + ns);
+      d.selfl = d.nbrl + nl;
       d.stage_max = c->cfg.stage_max == 0 ? kStageMax : c->cfg.stage_max;
     } catch (const Error &) {
       if (d.mixed) throw;
