@@ -119,6 +119,25 @@ def test_lengths_that_differ_gather_from_hbm():
     s.close()
 
 
+def test_lengths_made_uniform_after_init():
+    """A context made with lengths that differ and then given uniform ones:
+    the passes of a context uniform from the start, bit for bit."""
+    c = _case(500)
+    st, h = _state(c), c.h
+    want = _passes(c, st)
+    c.h = h * (1.0 - 0.05 * (np.arange(c.n) % 2))
+    s = cases.make_solver(c)
+    s.set("h", h)
+    for f, v in (("v", st["v"]), ("density", st["rho"]), ("sigma", st["sig"])):
+        s.set(f, v)
+    s.rebuild_neighbours()
+    for name, fields in PASSES:
+        s.eval(name)
+        for f in fields:
+            assert np.array_equal(s.get(f), want[f]), (f, name)
+    s.close()
+
+
 @pytest.mark.parametrize("opt", ["", "thermal", "plate"])
 def test_run_does_not_depend_on_staging(opt):
     """Steps with every tile from LDS, none, or those with small sets: the

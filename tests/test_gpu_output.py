@@ -69,3 +69,24 @@ def test_pack_before_init_fails():
     with pytest.raises(capi.WFError):
         s.pack_csv()
     s.close()
+
+
+def test_large_tables_match_host_packing():
+    """Tables of 20-50 MB, copied by several threads in chunks of 4 MiB whose
+    last is ragged: two calls in a row, with steps between them, against the
+    host packing of the same state."""
+    c = cases.cylinder_case("cyl_tables", 15e-3, 30e-3, 0.53e-3, 2700.0, 68.9e9, 0.3, cases.JC_AL, steps=1, jitter=1e-3,
+                            seed=3, v_top=-20.0, T0=300.0)
+    nf, nr = 4 * capi.XDMF_NF * c.n, 8 * capi.CSV_NCOL * c.n
+    print("n", c.n, "table MiB", nf / 2**20, nr / 2**20, flush=True)
+    assert min(nf, nr) > 16 << 20 and nf % (4 << 20) and nr % (4 << 20)
+    g = cases.make_solver(c, precision=capi.MIXED)
+    for steps in (3, 2):
+        g.step(steps)
+        g.sync()
+        f_h, iv_h, rows_h = output.table_from_fields(_host_fields(g))
+        f, iv = g.pack_xdmf()
+        assert np.array_equal(iv, iv_h)
+        assert np.array_equal(f, f_h)
+        assert np.array_equal(g.pack_csv(), rows_h)
+    g.close()

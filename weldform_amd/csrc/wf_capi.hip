@@ -466,11 +466,17 @@ DevMat to_dev(const wf_material &m) {
   return d;
 }
 
-// FP64: the passes from LDS take their smoothing length from the particle
-// itself, so every material's must be uniform; one or two lanes per particle
-// (asked for) leave too few wavefronts beside 60-120 KB of LDS per block and
-// gather from HBM
-void choose_f64(Ctx *c) {
+// h_uni (both precisions): every material's smoothing length is uniform.  The
+// conduction from LDS and the FP64 passes from LDS need it: they take the length
+// from the particle itself.  lds64: the FP64 passes from LDS; one or two lanes
+// per particle (asked for) leave too few wavefronts beside 60-120 KB of LDS per
+// block and gather from HBM.  Whether tiles are staged does not count: without
+// any staged (stage_max -1, no memory for the lists, lengths set uniform after
+// wf_init) the same kernels read HBM four lanes wide, a step of 1795 us at 954k
+// particles and 118 at 3.7k against 1796 and 134 of the two-lane gathers, and
+// 3353 against 3262 with 2h = 3 dx; there a third of the tiles still stage
+// (2783 us).
+void choose_passes(Ctx *c) {
   std::vector<double> hm(kMaxMat, -1.0);
   bool uni = true;
   for (int64_t i = 0; i < c->n; ++i) {
@@ -654,7 +660,7 @@ void allocate(Ctx *c) {
   // stage_cnt = -1 marks a tile that gathers from HBM
   c->list_alloc(d.stage_cnt, (size_t)d.ntiles);
   HIPCHK(hipMemsetAsync(d.stage_cnt, 0xff, sizeof(int) * (size_t)d.ntiles, c->st));
-  choose_f64(c);
+  choose_passes(c);
   // per-group sums: each material index's particles in internal order
   d.ngroups = 0;
   if (c->gsum_zone != -2) {
@@ -1410,7 +1416,7 @@ int wf_set_field(void *ctx, int32_t field, const double *h) {
         put_d4(c, d.xh[0], h, 3, 1, 1);
         put_d4(c, d.xh[1], h, 3, 1, 1);
         // the captured steps hold the pass the old lengths chose
-        choose_f64(c);
+        choose_passes(c);
         c->drop_graphs();
         break;
       case WF_F_V:

@@ -1086,7 +1086,9 @@ void launch_schedule(const Dev &d, hipStream_t st, int force, const BcTable *bc)
   k_schedule<<<rigid ? nblk(d.nrig) : 1, kBlock, 0, st>>>(d, force, rigid, bc ? *bc : BcTable{});
 }
 
-// rows built with kBuildLanes lanes per particle up to this many particles
+// rows built with kBuildLanes lanes per particle up to this many particles: the
+// whole search with 32 lanes against one 94 and 139 us at 1.3k, 107 and 138 at
+// 3.1k, 131 and 148 at 6.2k, 143 and 153 at 7.7k, and slower at 35k
 constexpr int kBuildWide = 8192;
 void launch_neighbours(const Dev &d, hipStream_t st, int cur) {
   k_cell_hist<<<nblk((long long)d.n + d.nrig), kBlock, 0, st>>>(d, cur);
@@ -2882,10 +2884,16 @@ WF_KERNEL void k_stress(Dev d, int buf, double dt) {
 
 // The stress update runs inside the rate kernel up to about one tile per CU:
 // there a launch costs more than what the update's dependent chain (return
-// map, powers) adds to each block.  Above, a kernel of its own keeps more of
-// those chains in flight.  Rates and update, fused against apart: 1.3k
-// particles 11.3 and 15.5 us, 35k 16.2 and 22.7; 56k (FP64) 26.6 and 32, but a
-// damage step 2 % slower; 370k 84 and 85, 954k 200 and 194 (FP64 301 and 272).
+// map, powers) adds to each block.  In large models a kernel of its own keeps
+// more of those chains in flight.  Whole yielding steps, fused against apart, us
+// (mixed; FP64; FP64 with damage):
+//   9k     79  81    81  83    79  82
+//   41k    95  99   109 113   111 115
+//   95k   116 120   156 160   162 166
+//   193k  165 166   224 222   235 230
+//   954k  625 616   954 918   964 908
+// so the line lies on the safe side: fused is 3 % faster up to about 100k
+// particles.
 constexpr int kFuseTiles = 320;
 bool launch_rates(const Dev &d, hipStream_t st, int buf, double dt, int do_stress) {
   if (d.ntiles > kFuseTiles) do_stress = 0;
