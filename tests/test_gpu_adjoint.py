@@ -17,8 +17,6 @@ difference with a 1e-4 relative parameter step (1e-5 with contact).
 Parameters differ in scale by ten orders, so components are compared as
 dL/d ln(theta) = theta dL/dtheta; one whose finite difference is below 1e-6
 of the largest is compared in absolute terms."""
-import ctypes
-
 import numpy as np
 import pytest
 
@@ -171,13 +169,6 @@ def test_window_loss_autograd():
     assert float(loss2) < float(loss.detach())
 
 
-def _free_bytes():
-    # (the library's own HIP runtime, found through its handle)
-    free, total = ctypes.c_size_t(0), ctypes.c_size_t(0)
-    assert capi.lib().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
-    return free.value
-
-
 def _small_window(stage_max):
     """A billet of soft metal in flow (several searches in the window) after 5 steps."""
     c = cases.config5_zone(steps=8, dx=0.72e-3, R=15e-3, L=30e-3, v_top=-5.0, seed=3)
@@ -193,21 +184,6 @@ def _small_window(stage_max):
 def _window_gradient(g):
     loss, hist = g.adj_forward(np.full(8, 1e4), checkpoint_every=4, kind=capi.ADJ_ZONE, index=3, component=2)
     return [loss, hist, g.adj_backward()] + [g.adj_field(f) for f in ("x", "v", "density", "sigmay", "pl_strain")]
-
-
-def test_window_storage_holds_no_staging_lists():
-    """The lists of the LDS passes follow from the neighbour rows: a window's
-    snapshots and tape take the device memory they take without them (20 MB a
-    copy here, seven copies)."""
-    used = {}
-    for stage_max in (-1, 0):
-        g = _small_window(stage_max)
-        free = _free_bytes()
-        _window_gradient(g)
-        used[stage_max] = (free - _free_bytes()) / 2**20
-        print("window MiB", used[stage_max], flush=True)
-        g.close()
-    assert abs(used[0] - used[-1]) < 16
 
 
 def test_gradient_does_not_depend_on_staging():

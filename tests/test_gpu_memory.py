@@ -1,7 +1,8 @@
 """FP64 contexts on a device whose memory is short: the staging lists of the
-passes from LDS are done without, or given back, where something that a
-context cannot do without asks for their memory.  The passes then read the
-same records from HBM, so that the results are the same bit for bit."""
+passes from LDS, and the gradient tape's copies of them, are done without, or
+given back, where something that a context cannot do without asks for their
+memory.  The passes then read the same records from HBM, or lists formed
+again, so that the results are the same bit for bit."""
 import ctypes
 import math
 
@@ -64,36 +65,43 @@ def test_lists_are_given_back():
     _gradient(g)
     g.close()
     c = _case()
-    results = {}
-    used = {}
+    want, used = {}, {}
     for stage_max in (-1, 0):  # without and with lists, all the memory there
         before = _free()
         g = _solver(c, stage_max=stage_max)
-        used[stage_max] = before - _free()
-        results[stage_max] = [g.get("x"), g.get("sigma"), *g.pack_xdmf()]
+        used["context", stage_max] = before - _free()
+        want = dict(state=[g.get("x"), g.get("sigma")], table=g.pack_xdmf())
         before = _free()
-        results[stage_max] += _gradient(g)
-        used["window"] = before - _free()
+        want["gradient"] = _gradient(g)
+        used["window", stage_max] = before - _free()
         g.close()
-    lists = used[0] - used[-1]
+    need, lists = used["context", -1], used["context", 0] - used["context", -1]
+    window, half = used["window", -1], lists // 2
     table = 4 * (capi.XDMF_NF + capi.XDMF_NI) * c.n
-    print("n", c.n, "MiB: lists", lists >> 20, "window", used["window"] >> 20, "table", table >> 20, flush=True)
+    print("n", c.n, "MiB: lists", lists >> 20, "window", window >> 20, "table", table >> 20, flush=True)
     assert lists > 128 << 20 and table > 64 << 20
-    half = lists // 2
-    # the lists do not fit; the table, or the window, fits only in their place
+    assert abs(used["window", 0] - window - 2 * lists) < half  # two tape slots' lists
+    cases_ = (  # what the device's memory holds, beside the context, and what is asked of it
+        ("no lists", need + half, ()),
+        ("lists or table", need + lists + table // 2, ("table",)),
+        ("lists or window", need + lists + table + window - half, ("table", "gradient")),
+        ("lists and window", need + lists + table + window + half, ("table", "gradient")),
+        ("the tape's lists or table", need + 3 * lists + window + table // 2, ("gradient", "table", "gradient")))
     with _Fill(8 << 30):
-        for what, leave in (("init", used[-1] + half), ("table", used[0] + table // 2),
-                            ("window", used[0] + table + used["window"] - half)):
+        for what, leave, asked in cases_:
             with _Fill(leave):
                 print("case", what, "MiB left", _free() >> 20, flush=True)
                 g = _solver(c)
-                got = [g.get("x"), g.get("sigma")]
-                if what != "init":
-                    got += g.pack_xdmf()
-                if what == "window":
-                    got += _gradient(g)
+                got = [("state", [g.get("x"), g.get("sigma")])]
+                for a in asked:
+                    if a == "table":
+                        got.append((a, g.pack_xdmf()))
+                    else:
+                        got.append((a, _gradient(g)))
+                        g.adj_restore()
                 g.step(2)
                 g.sync()
                 g.close()
-            for k, a in enumerate(got):
-                assert np.array_equal(a, results[0][k]), (what, k)
+            for name, arrays in got:
+                for k, (a, b) in enumerate(zip(arrays, want[name])):
+                    assert np.array_equal(a, b), (what, name, k)

@@ -874,6 +874,12 @@ WF_KERNEL void k_tape_lists(Dev d, AdjSlot s, int force, int *ver, int slot) {
   copy(s.nbr, d.nbr, ng * np * 16);
   copy(s.nnb, d.nnb, np * 4);
   copy(s.id, d.id, np * 4);
+  if (d.nbrl && s.nbrl) {
+    copy(s.nbrl, d.nbrl, ng * np * 8);
+    copy(s.selfl, d.selfl, np * 2);
+    copy(s.stage, d.stage, (long long)d.ntiles * kStageMax * 4);
+    for (long long k = t0; k < d.ntiles; k += stride) s.stage_cnt[k] = d.stage_cnt[k];
+  }
   if (d.contact) {
     copy(s.ccnt, d.ccnt, np * 4);
     copy(s.cidx, d.cidx, (long long)kMaxContact * np * 4);

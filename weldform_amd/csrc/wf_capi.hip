@@ -134,9 +134,9 @@ struct Ctx {
     return (T *)p;
   }
   // The staging lists (k_stage's: d.stage, d.nbrl, d.selfl, and d.stage_cnt):
-  // a function of the neighbour rows, so no part of the adjoint's snapshots and
-  // tape.  FP64 contexts do without them where the device's memory is short:
-  // their passes then read the same records from HBM, with the same results.
+  // a function of the neighbour rows, so no part of the adjoint's snapshots.
+  // FP64 contexts do without them where the device's memory is short: their
+  // passes then read the same records from HBM, with the same results.
   template <class T>
   void list_alloc(T *&p, size_t count) {
     if (p) (void)hipFree(p);  // (an earlier wf_init that failed)
@@ -150,12 +150,23 @@ struct Ctx {
     d.nbrl = d.selfl = nullptr;
     d.stage_max = 0;
   }
-  // memory taken after wf_init
+  void free_tape_lists() {
+    for (AdjSlot &s : adj.slot) {
+      if (s.stage) (void)hipFree(s.stage);
+      s.stage = s.stage_cnt = nullptr;
+      s.nbrl = s.selfl = nullptr;
+    }
+  }
+  // memory taken after wf_init: the tape's copies of the lists give way to it,
+  // then the lists
   hipError_t later_malloc(void **p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipErrorOutOfMemory || d.mixed || !d.nbrl) return e;
     (void)hipGetLastError();
     if ((e = hipStreamSynchronize(st)) != hipSuccess) return e;
+    free_tape_lists();
+    if ((e = hipMalloc(p, bytes)) != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
     free_lists();
     drop_graphs();  // (the captured steps hold the lists)
     if ((e = hipMemsetAsync(d.stage_cnt, 0xff, sizeof(int) * (size_t)d.ntiles, st)) != hipSuccess) return e;
@@ -209,6 +220,7 @@ struct Ctx {
     for (auto &e : ev_pool) (void)hipEventDestroy(e);
     for (auto &p : allocs) (void)hipFree(p.first);
     free_lists();
+    free_tape_lists();
     if (d.stage_cnt) (void)hipFree(d.stage_cnt);
     for (void *p : adj.mem) (void)hipFree(p);
     if (outbuf) (void)hipFree(outbuf);
@@ -1251,7 +1263,9 @@ void adj_prepare(Ctx *c, int k, size_t ncp) {
   A.snap_bytes = bytes;
   while (A.ckpt.size() < ncp) A.ckpt.push_back(c->adj_alloc<char>(bytes));
   A.ckh.resize(A.ckpt.size());
-  if (A.seg != k) {
+  const bool fresh = A.seg != k;
+  if (fresh) {
+    c->free_tape_lists();
     A.slot.clear();
     for (int s = 0; s <= k; ++s) A.slot.push_back(alloc_slot(c, s < k));
     A.ver = c->adj_alloc<int>((size_t)k);
@@ -1274,6 +1288,24 @@ void adj_prepare(Ctx *c, int k, size_t ncp) {
     b.thb = c->adj_alloc<double>((size_t)kAdjParams * np);
     b.part = c->adj_alloc<double>((size_t)kAdjParams * c->d.nblocks);
     A.grad = c->adj_alloc<double>(kAdjParams);
+  }
+  if (fresh && c->d.nbrl) {
+    // the staging lists of each slot's rows, last: what the tape can do without
+    const size_t np = (size_t)c->npad, nt = (size_t)c->d.ntiles;
+    const size_t ns = nt * kStageMax, nl = (size_t)nb_rows(c->cfg.max_nb) * np;
+    for (int s = 0; s < k; ++s) {
+      AdjSlot &q = A.slot[s];
+      if (hipMalloc((void **)&q.stage, (ns + nt) * sizeof(int) + (nl + np) * sizeof(uint16_t)) != hipSuccess) {
+        (void)hipGetLastError();
+        q.stage = nullptr;
+        c->free_tape_lists();
+        break;
+      }
+      // (np is a multiple of kBlock: every part but the counts starts 256-byte aligned)
+      q.nbrl = reinterpret_cast<uint16_t *>(q.stage + ns);
+      q.selfl = q.nbrl + nl;
+      q.stage_cnt = reinterpret_cast<int *>(q.selfl + np);
+    }
   }
 }
 
@@ -2462,14 +2494,21 @@ int wf_adj_backward(void *ctx, double *grad) {
       }
       tape_state(c, A.slot[len], c->cur);
       const auto ver = dget(c, A.ver, (size_t)len);
-      // reverse sweep over the segment; the staging lists follow the rows of
-      // the step in hand (at first the replay's last)
+      // reverse sweep over the segment.  The staging lists of the step's rows
+      // are the tape's, or formed again in the context's own (which hold those
+      // of the replay's last rows)
+      Dev dv = d;
       int staged = -1;
       for (int s = len - 1; s >= 0; --s) {
         AdjSlot s0 = A.slot[s];
         int v = s;
         while (v > 0 && !ver[v]) --v;
-        if (staged >= 0 && v != staged) {
+        if (d.nbrl && A.slot[v].nbrl) {
+          dv.stage = A.slot[v].stage;
+          dv.stage_cnt = A.slot[v].stage_cnt;
+          dv.nbrl = A.slot[v].nbrl;
+          dv.selfl = A.slot[v].selfl;
+        } else if (staged >= 0 && v != staged) {
           Dev rows = d;
           rows.nbr = A.slot[v].nbr;
           rows.nnb = A.slot[v].nnb;
@@ -2487,7 +2526,7 @@ int wf_adj_backward(void *ctx, double *grad) {
         if (A.cfg.loss_kind == WF_ADJ_PLANE) seeds.cf[A.cfg.loss_index][A.cfg.loss_component] = g;
         else seeds.react[zslot][A.cfg.loss_component] = g;
         const double kick = (A.step0 + n == 0) ? 0.5 * c->dt : c->dt;
-        launch_adj_step(d, c->st, s0, A.slot[s + 1], b, c->bc, seeds, c->dt, kick, A.cfg.material);
+        launch_adj_step(dv, c->st, s0, A.slot[s + 1], b, c->bc, seeds, c->dt, kick, A.cfg.material);
       }
       HIPCHK(hipGetLastError());
     }

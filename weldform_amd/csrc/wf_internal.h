@@ -338,6 +338,9 @@ struct AdjSlot {
   double4 *apre;               // acceleration after the pair pass (before contact)
   double *drho, *sr, *rr;      // density rate, strain rate [6], rotation rate [3]
   int *nbr, *nnb;              // neighbour list in effect
+  // and its staging lists, where the memory is there (else formed again)
+  int *stage, *stage_cnt;
+  uint16_t *nbrl, *selfl;
   int *cidx, *ccnt, *id;       // contact partners and particle ids in effect
   double4 *node, *enorm, *rv;  // rigid planes at the step's contact evaluation
 };
