@@ -50,6 +50,25 @@ def test_rows_match_brute_force(n, precision):
     assert s.neighbour_stats() == (2 * len(want), nb.max())
 
 
+@pytest.mark.parametrize("n", [577, 2048, 2049])
+def test_rows_of_a_plate_match_brute_force(n):
+    """Plane strain: many lanes per particle up to 2,048 particles."""
+    rng = np.random.default_rng(n)
+    k = np.arange(n)
+    c = cases.plate2d_small(steps=1)
+    c.x = np.stack([k % 48 * 1.0e-3, k // 48 * 1.0e-3, np.zeros(n)], axis=1)
+    c.x[:, :2] += rng.uniform(-2e-4, 2e-4, (n, 2))
+    for f in ("h", "mass", "density", "ids", "material", "sigmay", "T"):
+        setattr(c, f, np.resize(getattr(c, f), n))
+    print("n", n, flush=True)
+    s = cases.make_solver(c)
+    s.rebuild_neighbours()
+    want = _brute(c)
+    want = want[np.lexsort((want[:, 1], want[:, 0]))]
+    assert np.array_equal(s.neighbour_pairs(), want)
+    assert np.array_equal(s.get_int("nb"), np.bincount(want.ravel(), minlength=n))
+
+
 @pytest.mark.parametrize("n", [3001, 8193])
 def test_overfull_row_is_reported(n):
     s = cases.make_solver(_case(n), max_nb=40)

@@ -1088,8 +1088,10 @@ void launch_schedule(const Dev &d, hipStream_t st, int force, const BcTable *bc)
 
 // rows built with kBuildLanes lanes per particle up to this many particles: the
 // whole search with 32 lanes against one 94 and 139 us at 1.3k, 107 and 138 at
-// 3.1k, 131 and 148 at 6.2k, 143 and 153 at 7.7k, and slower at 35k
-constexpr int kBuildWide = 8192;
+// 3.1k, 131 and 148 at 6.2k, 143 and 153 at 7.7k, and slower at 35k.  Plane
+// strain has a third of the candidates, for which 32 lanes are mostly idle: 67
+// and 78 us at 1.1k, 73 and 77 at 2.1k, but 88 and 77 at 4.6k, 110 and 77 at 8.1k.
+constexpr int kBuildWide = 8192, kBuildWide2d = 2048;
 void launch_neighbours(const Dev &d, hipStream_t st, int cur) {
   k_cell_hist<<<nblk((long long)d.n + d.nrig), kBlock, 0, st>>>(d, cur);
   k_scan<<<scan_chunks(d.sncells) + (d.nrig ? scan_chunks(d.ncells) : 0), kScanThreads, 0, st>>>(d);
@@ -1104,7 +1106,7 @@ void launch_neighbours(const Dev &d, hipStream_t st, int cur) {
     const int g = nblk((long long)(d.sncells + group - 1) / group * 64);
     k_cell_sort<<<g < kSortBlocks ? g : kSortBlocks, kBlock, 0, st>>>(d, cur, group);
   }
-  if (d.n <= kBuildWide) k_build_nbr_wide<<<nblk((long long)d.n * kBuildLanes), kBlock, 0, st>>>(d, cur);
+  if (d.n <= (d.dim == 2 ? kBuildWide2d : kBuildWide)) k_build_nbr_wide<<<nblk((long long)d.n * kBuildLanes), kBlock, 0, st>>>(d, cur);
   else k_build_nbr<<<nblk(d.n), kBlock, 0, st>>>(d, cur);
   if (d.stage_max > 0) k_stage<<<d.ntiles < 2048 ? d.ntiles : 2048, kStageThreads, 0, st>>>(d, 0);
 }
