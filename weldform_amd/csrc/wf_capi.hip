@@ -500,6 +500,8 @@ void choose_passes(Ctx *c) {
   c->d.lds64 = !c->d.mixed && uni && (c->cfg.lanes == 0 || c->cfg.lanes == kLanesLds64);
 }
 
+constexpr int64_t kListless2d = 100000;  // see the staging lists
+
 void allocate(Ctx *c) {
   Dev &d = c->d;
   const size_t np = (size_t)c->npad;
@@ -711,8 +713,12 @@ void allocate(Ctx *c) {
       d.gc_hist = c->alloc<double>((size_t)d.ghist_cap * ng * kMaxMesh * 3);
     }
   }
-  // the staging lists last: what FP64 can do without
-  if (c->cfg.stage_max >= 0 && (d.mixed || d.lds64)) {
+  // The staging lists last: what FP64 can do without.  Plane strain with a
+  // search every step does: forming them costs more than its short rows gain
+  // (5.2k particles 96 us per yielding step with lists, 86 without; 20k 103 and
+  // 89; 60k 140 and 129), until the passes are long (201k 246 and 253).
+  const bool lists64 = d.lds64 && !(d.dim == 2 && c->cfg.ts_nb_inc == 1 && c->n <= kListless2d);
+  if (c->cfg.stage_max >= 0 && (d.mixed || lists64)) {
     try {
       // (np is a multiple of kBlock: every part starts 256-byte aligned)
       const size_t ns = (size_t)d.ntiles * kStageMax, nl = (size_t)nb_rows(c->cfg.max_nb) * np;
